@@ -1,11 +1,21 @@
 // Router and dispatch kernels (engine/ops.cu:137-423): router logits, per-block sigmoid+bias scoring with the
 // block expert pool and per-token top-K, routing weights, and the deterministic counting sort of (token, k)
 // pairs into expert-major slots with the GEMM work items. All counts stay on the device.
+#include <type_traits>
+
 #include "decode_plan.h"
 
 namespace llmoe {
 
 namespace {
+
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
 
 constexpr int MAXB = 32;    // tokens per routing block (one 32-bit token mask per expert)
 constexpr int MAXE = 256;   // experts (one thread each)
@@ -13,9 +23,7 @@ constexpr int PLAN_NT = 1024;          // planner threads: 4 per expert
 constexpr int MAXB_BLOCKS = 128;       // routing blocks whose masks the planner holds in registers (32 per thread)
 
 // logits partial c: fma chain over k = c H/8 .. (c+1) H/8 - 1 ascending from 0 (the summation order is fixed so
-// the CPU checker reproduces it). Workgroup tile: TT tokens x EW experts of one K chunk, the chunk's x slice and
-// its Wr slice (transposed, k contiguous per expert) staged in LDS, KS of k at a time; each thread runs one chain
-// per (token, expert) it owns. grid (E/EW, ceil(T/TT), 8).
+// the CPU checker reproduces it).
 // With q != nullptr the workgroups also write the A8 of the x slice (two 128-groups per token, the same operations
 // as quant_a8_kernel, spread over the expert slices), so the layer input is quantised without a launch of its own.
 __device__ __forceinline__ uint32_t okey(float v) {        // order-preserving unsigned image of a float
@@ -24,128 +32,195 @@ __device__ __forceinline__ uint32_t okey(float v) {        // order-preserving u
 }
 
 constexpr int RKW = 256;                                          // K per chunk (H = 2048)
-template <int KS>
-constexpr int router_stride() { return KS + 4; }                  // LDS row stride of the x and Wr slices
-template <int TT, int EW, int KS>
-constexpr int router_lds() { return (TT + EW) * router_stride<KS>() * 4; }
-// Tiles: <32 tokens, 8 experts, 256 threads> (one chain per thread: the decode step, latency-bound) and
-// <64 tokens, 64 experts, 512 threads> (2 tokens x 4 experts per thread: x and Wr reloaded 8x less from L2). The
-// chunk's K is staged KS at a time (the chains continue across the sub-chunks, so the order is the chunk's k
-// ascending either way): KS = 128 keeps the large tile's LDS at 66 KiB, two workgroups per CU (at 512 tokens
-// 20.0 -> 19.4 us per router stage, at 2048 tokens 66 -> 53 us, against one 133 KiB stage of 256 k). 4 tokens x 4
-// experts per thread (half the LDS reads per fma, one wave per SIMD) measured 23 us at 512 tokens.
-template <int TT, int EW, int NT, int TPT, int KS>
-__global__ void __launch_bounds__(NT) router_logits_kernel(const float* __restrict__ x, const float* __restrict__ Wr,
-                                                           int T, int H, int E, float* __restrict__ part,
-                                                           int8_t* __restrict__ q, float* __restrict__ qs,
-                                                           int* __restrict__ qsum) {
-    constexpr int EPT = TT * EW / NT / TPT;                      // chains per thread: TPT x EPT
-    constexpr int EG = EW / EPT;                                 // expert groups (threads per token group)
-    constexpr int RS = router_stride<KS>(), K4 = KS / 4;
-    constexpr int XV = TT * K4 / NT, WV = KS * (EW / 4) / NT;
-    static_assert(XV * NT == TT * K4 && WV * NT == KS * (EW / 4) && TPT * EPT * NT == TT * EW && RKW % KS == 0 &&
-                  KS % 128 == 0, "router tile");
+
+// Decode (T <= 32): workgroup tile 32 tokens x 8 experts of one K chunk, the chunk's x slice and its Wr slice
+// (transposed, k contiguous per expert) staged in LDS; each of the 256 threads runs one chain. grid E/8 x 8 chunks.
+// The step is latency-bound: 8 experts per workgroup put 256 workgroups on the chip (7.0 -> 5.8 us against 16 experts
+// and two chains per thread).
+constexpr int RD_EW = 8;                                          // experts per workgroup
+constexpr int RD_STRIDE = RKW + 4;                                // LDS row stride of the x and Wr slices
+constexpr int RD_LDS = (32 + RD_EW) * RD_STRIDE * 4;
+__global__ void __launch_bounds__(256) router_decode_kernel(const float* __restrict__ x, const float* __restrict__ Wr,
+                                                            int T, int H, int E, float* __restrict__ part,
+                                                            int8_t* __restrict__ q, float* __restrict__ qs,
+                                                            int* __restrict__ qsum) {
+    constexpr int RS = RD_STRIDE, K4 = RKW / 4, XV = 32 * K4 / 256, WV = RKW * (RD_EW / 4) / 256;
     extern __shared__ __align__(16) float rl[];
-    float* xs = rl;                       // [TT][RS]
-    float* ws = rl + TT * RS;             // [EW][RS]: Wr slice transposed, k contiguous per expert
-    // XCD-aware: workgroups go round-robin over the 8 XCDs by linear workgroup id.
-    // - Above 32 tokens, K chunk c = id % 8 puts every workgroup of chunk c on XCD c: the chunk's Wr rows and x
-    //   columns are fetched into that XCD's L2 only (512 tokens: 19.1 -> 17.9 us per router stage).
-    // - At decode (8 experts per slice), slice (id % 8) X/8 + (id / 8) % (X/8) puts the 4 slices of a 128-byte Wr
-    //   row segment on one XCD (config 1: 0.0545 -> 0.0539 ms per step; chunk per XCD: 0.0540 ms).
-    static_assert(ROUTER_KC == 8, "one K chunk per XCD");
-    const int X = gridDim.x;
-    const int id = blockIdx.x + X * (blockIdx.y + gridDim.y * blockIdx.z);
-    int c, sl, ty;
-    if (EW == 8 && X % 8 == 0) {
-        sl = (id % 8) * (X / 8) + (id / 8) % (X / 8);
-        const int r = id / X;
-        c = r % ROUTER_KC;
-        ty = r / ROUTER_KC;
-    } else {
-        c = id % ROUTER_KC;
-        sl = (id / ROUTER_KC) % X;
-        ty = id / ROUTER_KC / X;
+    float* xs = rl;                       // [32][RS]
+    float* ws = rl + 32 * RS;             // [8][RS]: Wr slice transposed, k contiguous per expert
+    // XCD-aware: workgroups go round-robin over the 8 XCDs by linear workgroup id; slice (id % 8) X/8 + (id / 8) %
+    // (X/8) puts the 4 slices of a 128-byte Wr row segment on one XCD (config 1: 0.0545 -> 0.0539 ms per step; chunk
+    // per XCD: 0.0540 ms). E % 64 == 0, so X % 8 == 0.
+    const int X = gridDim.x, id = blockIdx.x + X * blockIdx.z;
+    const int sl = (id % 8) * (X / 8) + (id / 8) % (X / 8), c = id / X;
+    const int e0 = sl * RD_EW, kb = c * RKW, tid = threadIdx.x;
+    float4 xv[XV], wv[WV];
+#pragma unroll
+    for (int i = 0; i < XV; ++i) {                                // x: 32 x 256 floats as float4
+        const int idx = tid + 256 * i, t = idx / K4, k4 = idx % K4;
+        xv[i] = t < T ? *reinterpret_cast<const float4*>(x + size_t(t) * H + kb + 4 * k4)
+                      : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
-    const int e0 = sl * EW, t0 = ty * TT;
-    const int tid = threadIdx.x;
-    // thread (token group tg, expert group eg): tokens tg TPT + i, experts j EG + eg (consecutive rows of the Wr
-    // slice across a wave's lanes: conflict-free), one fma chain each over the chunk's k ascending
-    const int tg = tid / EG, eg = tid % EG;
-    float acc[TPT][EPT];
 #pragma unroll
-    for (int i = 0; i < TPT; ++i)
+    for (int i = 0; i < WV; ++i) {                                // Wr: 256 x 8 floats as float4
+        const int idx = tid + 256 * i, k = idx / (RD_EW / 4), e4 = idx % (RD_EW / 4);
+        wv[i] = *reinterpret_cast<const float4*>(Wr + size_t(kb + k) * E + e0 + 4 * e4);
+    }
 #pragma unroll
-        for (int j = 0; j < EPT; ++j) acc[i][j] = 0.0f;
-    for (int h = 0; h < RKW / KS; ++h) {
-        const int kb = c * RKW + h * KS;
-        float4 xv[XV], wv[WV];
+    for (int i = 0; i < XV; ++i) {
+        const int idx = tid + 256 * i, t = idx / K4, k4 = idx % K4;
+        *reinterpret_cast<float4*>(xs + t * RS + 4 * k4) = xv[i];
+    }
 #pragma unroll
-        for (int i = 0; i < XV; ++i) {                            // x: TT x KS floats as float4
-            const int idx = tid + NT * i, t = idx / K4, k4 = idx % K4;
-            xv[i] = t0 + t < T ? *reinterpret_cast<const float4*>(x + size_t(t0 + t) * H + kb + 4 * k4)
-                               : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i = 0; i < WV; ++i) {
+        const int idx = tid + 256 * i, k = idx / (RD_EW / 4), e4 = idx % (RD_EW / 4);
+        ws[(4 * e4 + 0) * RS + k] = wv[i].x;
+        ws[(4 * e4 + 1) * RS + k] = wv[i].y;
+        ws[(4 * e4 + 2) * RS + k] = wv[i].z;
+        ws[(4 * e4 + 3) * RS + k] = wv[i].w;
+    }
+    __syncthreads();
+    // thread (token tid / 8, expert tid % 8)
+    const int t = tid / RD_EW, e = tid % RD_EW;
+    float acc = 0.0f;
+#pragma unroll 4
+    for (int k = 0; k < RKW; k += 4) {
+        const float4 a = *reinterpret_cast<const float4*>(xs + t * RS + k);
+        const float4 b = *reinterpret_cast<const float4*>(ws + e * RS + k);
+        acc = __builtin_fmaf(a.x, b.x, acc);
+        acc = __builtin_fmaf(a.y, b.y, acc);
+        acc = __builtin_fmaf(a.z, b.z, acc);
+        acc = __builtin_fmaf(a.w, b.w, acc);
+    }
+    if (q != nullptr) {
+        // A8 of the chunk's x slice (2 groups per token): 32 lanes per token, 2 tokens per wave job; wave w of expert
+        // slice b takes jobs w X + b, ...
+        const int lane = tid & 63;
+        for (int j = (tid >> 6) * X + sl; j < 16; j += 4 * X) {
+            const int tt = 2 * j + lane / 32, l = lane % 32;
+            const float4 a = *reinterpret_cast<const float4*>(xs + tt * RS + 8 * l);
+            const float4 b = *reinterpret_cast<const float4*>(xs + tt * RS + 8 * l + 4);
+            const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            const size_t gi = size_t(tt) * (H / GROUP) + kb / GROUP + (l >> 4);   // (rows beyond T are not written)
+            quant_a8_8(v, lane, q + size_t(tt) * H + kb + 8 * l, qs + gi, qsum + gi, tt < T);
         }
+    }
+    if (t < T) part[(size_t(c) * T + t) * E + e0 + e] = acc;
+}
+
+// Above 32 tokens: the chains on the matrix cores. v_mfma_f32_16x16x4_f32 accumulates its four k in ascending order
+// with one rounding each -- bit for bit the fma chain (checked on the device against the CPU chain, subnormals
+// included; the GPU tests compare the partials' sums with the checker's) -- at twice the vector fma rate: 1024 fma
+// in 32 cycles per SIMD. Tile: 32 M tokens x 32 M experts of one K chunk, 4 waves of M x M 16x16 MFMA tiles. The K
+// chunk runs in stages of 64 k: the x slice goes through LDS (two buffers) as [token][k % 4][k / 4], so that a lane
+// reads the k of four MFMAs (its k are congruent mod 4) as 16 bytes (row stride 68: conflict-free); Wr operands come
+// straight from global memory (64 contiguous bytes per k). A stage's loads are in flight during the stage before.
+// Experts are the MFMA rows, so a lane ends with four consecutive experts of one token.
+// What bounds it: the f32 MFMA issue (28 us of 4096 tokens' 59 at 2.4 GHz; vector work does not overlap f32 MFMAs, so
+// the A8 and the addressing add to it). Against vector fma chains on 64 x 64 tiles in LDS: 15.1 -> 10.5 us at 512
+// tokens, 93 -> 59 us at 4096.
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int RM_KS = 64, RM_STRIDE = RM_KS + 4;
+template <int M>
+constexpr int rm_lds() { return 2 * 32 * M * RM_STRIDE * 4; }
+template <int M>
+__global__ void __launch_bounds__(256, 4) router_mfma_kernel(const float* __restrict__ x, const float* __restrict__ Wr,
+                                                             int T, int H, int E, float* __restrict__ part,
+                                                             int8_t* __restrict__ q, float* __restrict__ qs,
+                                                             int* __restrict__ qsum) {
+    constexpr int TT = 32 * M, RS = RM_STRIDE, K4 = RM_KS / 4, XV = TT * K4 / 256, NJ = RM_KS / 4, QS = RM_KS / 4;
+    constexpr int NH = RKW / RM_KS;
+    static_assert(2 * RM_KS == GROUP && NH % 2 == 0, "a 128-group is two stages");
+    extern __shared__ __align__(16) float xs[];                   // [2][TT][RS]: [k % 4][k / 4] per token
+    // XCD-aware: workgroups go round-robin over the 8 XCDs by linear id, so K chunk c = id % 8 keeps the chunk's Wr
+    // rows and x columns in one XCD's L2
+    static_assert(ROUTER_KC == 8, "one K chunk per XCD");
+    const int X = gridDim.x, id = blockIdx.x + X * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int c = id % ROUTER_KC, sl = (id / ROUTER_KC) % X, ty = id / ROUTER_KC / X;
+    const int e0 = sl * TT, t0 = ty * TT;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, q4 = lane >> 4;
+    const int te = 16 * M * (w & 1), tt0 = 16 * M * (w >> 1);     // the wave's experts and tokens inside the tile
+    // this thread's x elements of a stage (rows beyond T read the last row; their outputs are not stored)
+    const float* xp[XV];
+    float* xl[XV];
 #pragma unroll
-        for (int i = 0; i < WV; ++i) {                            // Wr: KS x EW floats as float4
-            const int idx = tid + NT * i, k = idx / (EW / 4), e4 = idx % (EW / 4);
-            wv[i] = *reinterpret_cast<const float4*>(Wr + size_t(kb + k) * E + e0 + 4 * e4);
-        }
-        if (h > 0) __syncthreads();                               // the previous sub-chunk has been read
+    for (int i = 0; i < XV; ++i) {
+        const int idx = tid + 256 * i, t = idx / K4, k4 = idx % K4;
+        xp[i] = x + size_t(min(t0 + t, T - 1)) * H + c * RKW + 4 * k4;
+        xl[i] = xs + t * RS + k4;
+    }
+    const float* wp = Wr + size_t(c * RKW + q4) * E + e0 + te + r;
+    float4 xv[XV];
+    float wv[2][M][NJ];
+    auto load = [&](auto hc) {
+        constexpr int h = decltype(hc)::value;
+#pragma unroll
+        for (int i = 0; i < XV; ++i) xv[i] = *reinterpret_cast<const float4*>(xp[i] + h * RM_KS);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int i = 0; i < M; ++i) wv[h & 1][i][j] = wp[size_t(h * RM_KS + 4 * j) * E + 16 * i];
+    };
+    v4f acc[M][M];                                                // [expert tile][token tile]
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int j = 0; j < M; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    load(std::integral_constant<int, 0>{});
+    static_for<0, NH>([&](auto hc) {
+        constexpr int h = decltype(hc)::value;
+        float* buf = xs + (h & 1) * TT * RS;
 #pragma unroll
         for (int i = 0; i < XV; ++i) {
-            const int idx = tid + NT * i, t = idx / K4, k4 = idx % K4;
-            *reinterpret_cast<float4*>(xs + t * RS + 4 * k4) = xv[i];
+            float* p = xl[i] + (h & 1) * TT * RS;
+            p[0] = xv[i].x;
+            p[QS] = xv[i].y;
+            p[2 * QS] = xv[i].z;
+            p[3 * QS] = xv[i].w;
         }
+        __syncthreads();   // (also: the readers of the other buffer, which the next stage overwrites, are done)
+        if constexpr (h + 1 < NH) load(std::integral_constant<int, h + 1>{});
 #pragma unroll
-        for (int i = 0; i < WV; ++i) {
-            const int idx = tid + NT * i, k = idx / (EW / 4), e4 = idx % (EW / 4);
-            ws[(4 * e4 + 0) * RS + k] = wv[i].x;
-            ws[(4 * e4 + 1) * RS + k] = wv[i].y;
-            ws[(4 * e4 + 2) * RS + k] = wv[i].z;
-            ws[(4 * e4 + 3) * RS + k] = wv[i].w;
+        for (int j = 0; j < NJ; j += 4) {
+            float4 xa[M];
+#pragma unroll
+            for (int i = 0; i < M; ++i)
+                xa[i] = *reinterpret_cast<const float4*>(buf + (tt0 + 16 * i + r) * RS + q4 * QS + j);
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+                for (int i = 0; i < M; ++i)
+#pragma unroll
+                    for (int n = 0; n < M; ++n) {
+                        const float xk = jj == 0 ? xa[n].x : jj == 1 ? xa[n].y : jj == 2 ? xa[n].z : xa[n].w;
+                        acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[h & 1][i][j + jj], xk, acc[i][n], 0, 0, 0);
+                    }
         }
-        __syncthreads();
-#pragma unroll 4
-        for (int k = 0; k < KS; k += 4) {
-            float4 a[TPT], b[EPT];
+        if constexpr (h & 1) {
+            if (q != nullptr) {
+                // A8 of the 128-group now in the two buffers: 16 lanes per token, 4 tokens per wave job; wave w of expert
+                // slice b takes jobs w X + b, ...
+                const int kb = c * RKW + (h - 1) * RM_KS;
+                for (int j = w * X + sl; j < TT / 4; j += 4 * X) {
+                    const int tl = 4 * j + q4, t = t0 + tl;
+                    const float* v0 = xs + (r >> 3) * TT * RS + tl * RS + 2 * (r & 7);
+                    float v[8];
 #pragma unroll
-            for (int i = 0; i < TPT; ++i) a[i] = *reinterpret_cast<const float4*>(xs + (tg * TPT + i) * RS + k);
-#pragma unroll
-            for (int j = 0; j < EPT; ++j) b[j] = *reinterpret_cast<const float4*>(ws + (j * EG + eg) * RS + k);
-#pragma unroll
-            for (int i = 0; i < TPT; ++i)
-#pragma unroll
-                for (int j = 0; j < EPT; ++j) {
-                    acc[i][j] = __builtin_fmaf(a[i].x, b[j].x, acc[i][j]);
-                    acc[i][j] = __builtin_fmaf(a[i].y, b[j].y, acc[i][j]);
-                    acc[i][j] = __builtin_fmaf(a[i].z, b[j].z, acc[i][j]);
-                    acc[i][j] = __builtin_fmaf(a[i].w, b[j].w, acc[i][j]);
+                    for (int i = 0; i < 8; ++i) v[i] = v0[(i & 3) * QS + (i >> 2)];
+                    const size_t gi = size_t(t) * (H / GROUP) + kb / GROUP;   // (rows beyond T are not written)
+                    quant_a8_8(v, lane, q + size_t(t) * H + kb + 8 * r, qs + gi, qsum + gi, t < T);
                 }
-        }
-        if (q != nullptr) {
-            // A8 of the sub-chunk's x slice (KS / 128 groups per token): LPT = KS / 8 lanes per token, 8 values each,
-            // 64 / LPT tokens per wave job; wave w of expert slice b takes jobs w E/EW + b + i NWV E/EW, so the jobs
-            // are spread over the expert slices' workgroups
-            constexpr int NWV = NT / 64, LPT = KS / 8, TPW = 64 / LPT;
-            const int lane = tid & 63;
-            for (int j = (tid >> 6) * X + sl; j < TT / TPW; j += NWV * X) {
-                const int tt = TPW * j + lane / LPT, l = lane % LPT;
-                const float4 a = *reinterpret_cast<const float4*>(xs + tt * RS + 8 * l);
-                const float4 b = *reinterpret_cast<const float4*>(xs + tt * RS + 8 * l + 4);
-                const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-                const int t = t0 + tt;   // (rows beyond T: computed on zeros, not written)
-                const size_t gi = size_t(t) * (H / GROUP) + kb / GROUP + (l >> 4);
-                quant_a8_8(v, lane, q + size_t(t) * H + kb + 8 * l, qs + gi, qsum + gi, t < T);
+                if constexpr (h + 1 < NH) __syncthreads();   // both buffers have been read
             }
         }
-    }
+    });
 #pragma unroll
-    for (int i = 0; i < TPT; ++i) {
-        const int t = t0 + tg * TPT + i;
+    for (int n = 0; n < M; ++n) {
+        const int t = t0 + tt0 + 16 * n + r;
         if (t < T)
 #pragma unroll
-            for (int j = 0; j < EPT; ++j) part[(size_t(c) * T + t) * E + e0 + j * EG + eg] = acc[i][j];
+            for (int i = 0; i < M; ++i)
+                *reinterpret_cast<v4f*>(part + (size_t(c) * T + t) * E + e0 + te + 16 * i + 4 * q4) = acc[i][n];
     }
 }
 
@@ -671,24 +746,14 @@ __global__ void __launch_bounds__(256) place_kernel(const int* __restrict__ topk
 
 hipError_t launch_router_logits(const float* x, const float* Wr, int T, int H, int E, float* part, int8_t* q,
                                 float* qs, int* qsum, hipStream_t st) {
-    static bool attr = false;
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(router_logits_kernel<32, 8, 256, 1, 256>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, router_lds<32, 8, 256>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(router_logits_kernel<64, 64, 512, 2, 128>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, router_lds<64, 64, 128>());
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
     if (T <= 32) {
-        const dim3 grid(E / 8, 1, ROUTER_KC);
-        router_logits_kernel<32, 8, 256, 1, 256><<<grid, 256, router_lds<32, 8, 256>(), st>>>(x, Wr, T, H, E, part, q,
-                                                                                             qs, qsum);
+        router_decode_kernel<<<dim3(E / RD_EW, 1, ROUTER_KC), 256, RD_LDS, st>>>(x, Wr, T, H, E, part, q, qs, qsum);
+    } else if (T <= 256) {   // 32 x 32 tiles: at 256 tokens 512 workgroups (64 x 64: 128, half of the CUs)
+        router_mfma_kernel<1><<<dim3(E / 32, (T + 31) / 32, ROUTER_KC), 256, rm_lds<1>(), st>>>(x, Wr, T, H, E, part, q,
+                                                                                               qs, qsum);
     } else {
-        const dim3 grid(E / 64, (T + 63) / 64, ROUTER_KC);
-        router_logits_kernel<64, 64, 512, 2, 128><<<grid, 512, router_lds<64, 64, 128>(), st>>>(x, Wr, T, H, E, part,
-                                                                                                q, qs, qsum);
+        router_mfma_kernel<2><<<dim3(E / 64, (T + 63) / 64, ROUTER_KC), 256, rm_lds<2>(), st>>>(x, Wr, T, H, E, part, q,
+                                                                                               qs, qsum);
     }
     return hipGetLastError();
 }
