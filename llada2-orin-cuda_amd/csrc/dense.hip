@@ -2,8 +2,8 @@
 // the lm_head through the expert GEMM as one "expert" holding every token). One [R, 2048] matrix of b-bit codes
 // in packlib "i8", relaid out once for the MFMA kernels; a call multiplies T tokens' A8 rows by it:
 //     Y[t, r] (=|+=) sum_g fma chain of scale_w[r, g] scale_x[t, g] P_g[r, t]      (the expert GEMMs' epilogue)
-// T <= 32: the streamed kernel over items of 16 tokens x row blocks; T > 32: the tiled kernel over chunks of
-// <= 64 tokens, the (chunk, row block) tasks split evenly over its resident workgroups.
+// T <= 32: the split-K kernel; T > 32: the tiled kernel over chunks of <= 64 tokens, the (chunk, row block) tasks split
+// evenly over its resident workgroups. Neither needs work lists: an object holds nothing that a call writes.
 #include <cstdarg>
 #include <cstdio>
 #include <new>
@@ -15,13 +15,10 @@
 using namespace llmoe;
 
 struct llmoe_dense {
-    int R = 0, K = 0, bits = 0, max_tokens = 0, G = 0;
+    int R = 0, K = 0, bits = 0, max_tokens = 0;
     uint8_t* arena = nullptr;      // relaid-out matrix
     uint64_t* off = nullptr;       // [1] = 0 (the GEMMs' per-expert matrix offsets)
     int8_t* bits_d = nullptr;      // [1]
-    Item* units = nullptr;         // streamed units or tiled chunks of the latest call
-    int* n_units = nullptr;        // [1]
-    int* tstart = nullptr;         // [G + 1] tiled work partition
     std::vector<void*> allocs;
     ~llmoe_dense() {
         for (void* p : allocs) (void)hipFree(p);
@@ -45,20 +42,6 @@ int dfail(int code, const char* fmt, ...) {
         if (e_ != hipSuccess) return dfail(LLMOE_EHIP, "%s: %s", #expr, hipGetErrorString(e_));           \
     } while (0)
 
-// Work list of a tiled call (T > 32), one workgroup: chunks {0, j per, n, 0} and the partition of the nch nrb equal
-// (chunk, row block) tasks: workgroup w starts at task ceil(w N / G) (chunk | rb << TASK_RB_SHIFT).
-__global__ void __launch_bounds__(256) dense_plan_kernel(int T, int R, int bits, int G, Item* __restrict__ units,
-                                                         int* __restrict__ n_units, int* __restrict__ tstart) {
-    const int nch = tiled_chunks(T), per = tiled_per(T), nrb = R / (16 * tiled_waves(false) * tiled_spw(false, bits));
-    for (int j = threadIdx.x; j < nch; j += blockDim.x) units[j] = Item{0, j * per, min(per, T - j * per), 0};
-    const long long N = (long long)nch * nrb;
-    for (int w = threadIdx.x; w <= G; w += blockDim.x) {
-        const long long t = ((long long)w * N + G - 1) / G;
-        tstart[w] = int(t / nrb) | (int(t % nrb) << TASK_RB_SHIFT);
-    }
-    if (threadIdx.x == 0) n_units[0] = nch;
-}
-
 }  // namespace
 
 extern "C" {
@@ -80,20 +63,15 @@ int llmoe_dense_create(int rows, int k, int bits, const uint8_t* blob, size_t bl
     D->K = k;
     D->bits = bits;
     D->max_tokens = max_tokens;
-    D->G = tiled_grid(GEMM_DENSE);
     auto alloc = [&](void** p, size_t n) {
         if (hipMalloc(p, std::max<size_t>(n, 16)) != hipSuccess) return false;
         D->allocs.push_back(*p);
         return true;
     };
     uint8_t* staging = nullptr;
-    const size_t cap = size_t(tiled_chunks(max_tokens));
-    bool ok = D->G > 0 && alloc(reinterpret_cast<void**>(&D->arena), bytes) &&
+    bool ok = tiled_grid(GEMM_DENSE) > 0 && alloc(reinterpret_cast<void**>(&D->arena), bytes) &&
               alloc(reinterpret_cast<void**>(&D->off), sizeof(uint64_t)) &&
-              alloc(reinterpret_cast<void**>(&D->bits_d), 4) &&   // a whole dword: read by scalar dword loads
-              alloc(reinterpret_cast<void**>(&D->units), cap * sizeof(Item)) &&
-              alloc(reinterpret_cast<void**>(&D->n_units), sizeof(int)) &&
-              alloc(reinterpret_cast<void**>(&D->tstart), size_t(D->G + 1) * sizeof(int));
+              alloc(reinterpret_cast<void**>(&D->bits_d), 4);   // a whole dword: read by scalar dword loads
     if (!ok) {
         delete D;
         return dfail(LLMOE_ENOMEM, "device allocation");
@@ -127,16 +105,10 @@ int llmoe_dense_forward(llmoe_dense* D, const int8_t* xq, const float* xs, const
     if (T < 1 || T > D->max_tokens) return dfail(LLMOE_EINVAL, "T = %d outside [1, max_tokens = %d]", T, D->max_tokens);
     const hipStream_t st = static_cast<hipStream_t>(stream);
     const bool tiled = T > 32;
-    if (tiled) {   // (T <= 32: the split-K kernel needs no work list)
-        dense_plan_kernel<<<1, 256, 0, st>>>(T, D->R, D->bits, D->G, D->units, D->n_units, D->tstart);
-        DHIP(hipGetLastError());
-    }
     GemmArgs g{};
     g.base = D->arena;
     g.off = D->off;
     g.bits = D->bits_d;
-    g.items = D->units;
-    g.n_items = D->n_units;
     g.slot_token = nullptr;
     g.xq = xq;
     g.xs = xs;
@@ -144,7 +116,6 @@ int llmoe_dense_forward(llmoe_dense* D, const int8_t* xq, const float* xs, const
     g.K = D->K;
     g.R = D->R;
     g.Y = y;
-    g.tstart = D->tstart;
     g.accumulate = accumulate ? 1 : 0;
     g.dense_T = T;
     DHIP(tiled ? launch_tiled_gemm(GEMM_DENSE, g, st) : launch_dense_splitk(D->bits, g, st));

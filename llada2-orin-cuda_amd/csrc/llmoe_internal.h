@@ -351,7 +351,7 @@ struct GemmArgs {
     int32_t* P;                 // group-products out [n, R, K/128] (test entry)
     const int* tstart;          // tiled: [G + 1] first task of each workgroup (the work partition above)
     int accumulate;             // GEMM_DENSE: Y += acc instead of Y = acc
-    int dense_T;                // dense projection at T <= 32 (launch_dense_splitk): the tokens
+    int dense_T;                // dense projections: the tokens
     int fast;                   // gate_up: SiLU by the hardware exp / reciprocal and fp16 conversion
     // streamed down GEMM: with zin set, the B rows are staged as A8(FWHT-512(zin[slot])) instead of read from xq / xs /
     // xsum, and the units of row block 0 also write those rows to xq_out / xs_out / xsum_out
@@ -411,7 +411,7 @@ hipError_t launch_dense_splitk(int bits, const GemmArgs& a, hipStream_t st);
 // writes the plan's lists (DecodePlanArgs::d) for the down GEMM and the combine
 struct DecodePlanArgs;
 hipError_t launch_expert_gemm_plan(const GemmArgs& a, const DecodePlanArgs& p, hipStream_t st);
-// tiled units (a.items / a.n_items): mode GEMM_GATE_UP or GEMM_DOWN
+// mode GEMM_GATE_UP or GEMM_DOWN: tiled units (a.items, a.tstart); GEMM_DENSE: a.dense_T tokens, no lists
 hipError_t tiled_setup();
 // resident workgroups of the tiled GEMM grid for mode GEMM_GATE_UP / GEMM_DOWN (the G of the work partition)
 int tiled_grid(int mode);

@@ -488,7 +488,9 @@ __device__ __forceinline__ void tiled_body(const GemmArgs& a, const Item& it, co
 }
 
 // Workgroup w runs the row-block tasks tstart[w] .. tstart[w + 1] (chunk-major, so the chunk's activations are
-// staged once per run of its row blocks).
+// staged once per run of its row blocks). GEMM_DENSE has no lists: the dense_T tokens are equal chunks of one matrix, and
+// the workgroup's share of the equal (chunk, row block) tasks is a closed form evaluated here (a planning launch of its
+// own cost 3.5 us a projection).
 template <int MODE>
 __global__ void __launch_bounds__(nthreads_for(MODE == GEMM_DOWN ? 512 : 2048)) tiled_gemm(GemmArgs a) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -498,13 +500,33 @@ __global__ void __launch_bounds__(nthreads_for(MODE == GEMM_DOWN ? 512 : 2048)) 
     // hot expert -- listed one after another -- share that XCD's L2 for the expert's weights
     const int G = gridDim.x;
     const int p = G % NXCD ? int(blockIdx.x) : int(blockIdx.x % NXCD) * (G / NXCD) + int(blockIdx.x / NXCD);
-    const int s0 = *const_ptr(a.tstart + p), s1 = *const_ptr(a.tstart + p + 1);
-    const int c0 = s0 & CMASK, r0 = s0 >> TASK_RB_SHIFT, c1 = s1 & CMASK, r1 = s1 >> TASK_RB_SHIFT;
+    int c0, r0, c1, r1, dper = 0;
+    if constexpr (MODE == GEMM_DENSE) {
+        // tasks [ceil(p N / G), ceil((p + 1) N / G)) of N = chunks x row blocks (in 32 bits: p (N % G) < G^2)
+        const int bits = *const_ptr(reinterpret_cast<const int*>(a.bits)) << 24 >> 24;
+        const int nrb = a.R / (16 * tiled_waves(false) * tiled_spw(false, bits));
+        const int N = tiled_chunks(a.dense_T) * nrb, nq = N / G, nr = N % G;
+        const int s0 = p * nq + (p * nr + G - 1) / G, s1 = (p + 1) * nq + ((p + 1) * nr + G - 1) / G;
+        c0 = s0 / nrb;
+        r0 = s0 % nrb;
+        c1 = s1 / nrb;
+        r1 = s1 % nrb;
+        dper = tiled_per(a.dense_T);
+    } else {
+        const int s0 = *const_ptr(a.tstart + p), s1 = *const_ptr(a.tstart + p + 1);
+        c0 = s0 & CMASK;
+        r0 = s0 >> TASK_RB_SHIFT;
+        c1 = s1 & CMASK;
+        r1 = s1 >> TASK_RB_SHIFT;
+    }
     for (int c = c0; c < c1 || (c == c1 && r1 > 0); ++c) {
         // the chunk, and the expert's matrix offset and code width together, by scalar loads (the lists are
         // written by earlier kernels only)
-        const auto* ip = const_ptr(reinterpret_cast<const int*>(a.items + c));
-        const Item it{ip[0], ip[1], ip[2], ip[3]};
+        Item it{0, c * dper, min(dper, a.dense_T - c * dper), 0};
+        if constexpr (MODE != GEMM_DENSE) {
+            const auto* ip = const_ptr(reinterpret_cast<const int*>(a.items + c));
+            it = Item{ip[0], ip[1], ip[2], ip[3]};
+        }
         const uint64_t off = *const_ptr(a.off + it.expert);
         const uint32_t bw4 = *const_ptr(reinterpret_cast<const uint32_t*>(a.bits) + (it.expert >> 2));
         asm volatile("" ::"s"(off), "s"(bw4));
