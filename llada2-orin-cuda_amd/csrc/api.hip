@@ -111,6 +111,7 @@ struct llmoe_layer {
     size_t items_cap = 0;                           // work items (before the split into row blocks)
     size_t chunks_cap = 0;                          // tiled chunks
     int g_gu = 0, g_dn = 0;                         // tiled GEMM grids (workgroups of the work partition)
+    int max_gu = 0, max_dn = 0;                     // decode: the most units of a list that is split finer
     int* tstart = nullptr;                          // [g_gu + 1 + g_dn + 1] tiled work partition
     bool fast = false;                              // numerics: the gate_up SiLU by the hardware transcendentals
     // routing state
@@ -373,7 +374,7 @@ int llmoe_layer_create(const llmoe_layer_desc* desc, const void* blob, size_t bl
     L->items_cap = E + (Tm * K + 15) / 16 + (Tm + 15) / 16 + 2;
     ALLOC(L->units_gu, L->items_cap * MAX_UNITS_PER_ITEM);
     ALLOC(L->units_dn, L->items_cap * MAX_UNITS_PER_ITEM);
-    ALLOC(L->n_units, 4);
+    ALLOC(L->n_units, 6);   // gate_up / down units, tiled chunks (twice), the split of the two streamed lists
     L->chunks_cap = E + (Tm * K + TILED_NTOK - 1) / TILED_NTOK + (Tm + TILED_NTOK - 1) / TILED_NTOK + 2;
     if ((5 * L->chunks_cap + 2) * sizeof(uint32_t) > 65536)
         return bail(fail(LLMOE_EINVAL, "max_tokens = %d: more tiled chunks than the planner holds", int(Tm)));
@@ -382,6 +383,14 @@ int llmoe_layer_create(const llmoe_layer_desc* desc, const void* blob, size_t bl
     L->g_gu = tiled_grid(GEMM_GATE_UP);
     L->g_dn = tiled_grid(GEMM_DOWN);
     if (L->g_gu < 1 || L->g_dn < 1) return bail(fail(LLMOE_EHIP, "tiled GEMM occupancy query failed"));
+    // Decode units are split finer while they run in one round (gate_up), or at 5/4 units per CU (down: every unit
+    // transforms its item's Z rows again). us a layer, split against not: one token 31.4 / 43.2, 8 tokens (276 gate_up
+    // units -> 752, 138 down -> 276) 39.3 / 47.1, 32 tokens with the pool (280 -> 528, 140 -> 280) 42.9 / 50.4. Beyond:
+    // two rounds of gate_up units 43.9; 560 down units 43.6; 384 down units (4-bit experts, 192 unsplit) 42.9 / 42.5. The
+    // lists hold at least 64 MAX_UNITS_PER_ITEM units.
+    L->max_gu = std::min<long>(expert_grid(GEMM_GATE_UP), long(L->items_cap) * MAX_UNITS_PER_ITEM);
+    L->max_dn = std::min<long>(long(expert_grid(GEMM_DOWN)) * 5 / 12, long(L->items_cap) * MAX_UNITS_PER_ITEM);
+    if (L->max_gu < 1 || L->max_dn < 1) return bail(fail(LLMOE_EHIP, "GEMM occupancy query failed"));
     ALLOC(L->tstart, size_t(L->g_gu + L->g_dn + 2));
     ALLOC(L->slot_token, S);
     ALLOC(L->slot_weight, S);
@@ -445,7 +454,8 @@ int route_impl(llmoe_layer* L, const float* x, const float* logits, int T, hipSt
         HIPCHECK(launch_decode_route(part, nchunks, L->bias, T, d.n_experts, d.top_k, d.pool, d.routed_scale, L->sig,
                                      L->topk, L->topw, L->blockmax, L->tmask, d.has_shared, L->bits_d,
                                      L->count, L->start, L->units_gu, L->units_dn, L->n_units, L->slot_token,
-                                     L->slot_weight, L->tok_slots, qx, defer_dispatch ? 0 : 1, st));
+                                     L->slot_weight, L->tok_slots, L->max_gu, L->max_dn, qx,
+                                     defer_dispatch ? 0 : 1, st));
         L->mark(LLMOE_STAGE_ROUTE, true, st);
         L->routed_T = T;
         L->plan_pending = defer_dispatch;
@@ -503,6 +513,7 @@ int experts_impl(llmoe_layer* L, const int8_t* xq, const float* xs, const int32_
     // gate_up: B rows are token rows of x'
     g.items = L->units_gu;
     g.n_items = L->n_units;
+    g.fine = L->n_units + 4;
     g.off = L->gu_off_d;
     g.slot_token = L->slot_token;
     g.xq = xq; g.xs = xs; g.xsum = xsum;
@@ -523,7 +534,8 @@ int experts_impl(llmoe_layer* L, const int8_t* xq, const float* xs, const int32_
     if (plan) {
         const DecodePlanArgs pa{T, d.n_experts, K, L->tmask, L->tcopy, L->topk, L->topw,
                                 DispatchOut{d.has_shared, 16, L->bits_d, L->count, L->start, L->units_gu, L->units_dn,
-                                            L->n_units, L->slot_token, L->slot_weight, L->tok_slots},
+                                            L->n_units, L->slot_token, L->slot_weight, L->tok_slots, L->max_gu,
+                                            L->max_dn},
                                 L->d_off_d, DOWN_PF_BYTES};
         L->last_pa = pa;
         L->last_pa.tmask = L->tcopy;   // a re-launch plans from the copy
@@ -540,6 +552,7 @@ int experts_impl(llmoe_layer* L, const int8_t* xq, const float* xs, const int32_
     // down: B rows are slot rows of Z'
     g.items = L->units_dn;
     g.n_items = L->n_units + 1;
+    g.fine = L->n_units + 5;
     g.off = L->d_off_d;
     g.slot_token = nullptr;
     g.xq = w.zq; g.xs = w.zs; g.xsum = w.zsum;

@@ -10,6 +10,10 @@
 // Every workgroup of 256 threads can build the plan in LDS (one thread per expert: three scans), and any of them
 // can then name unit u of the gate_up list without the list in memory: the class from the class totals, the
 // expert by binary search on the class's inclusive scan, then the item and row block.
+//
+// Few units leave most of the chip idle while each streams its strips one after another, so the plan splits the units
+// of a list finer (half, a quarter of the strips per wave) as long as they still fit the resident workgroups in one
+// round (DispatchOut::max_gu, max_dn).
 #pragma once
 #include "llmoe_internal.h"
 
@@ -28,6 +32,7 @@ struct DispatchOut {         // the plan and placement written for the down GEMM
     int* slot_token;
     float* slot_weight;
     int* tok_slots;
+    int max_gu, max_dn;      // most units of a list that is split finer
 };
 
 struct DecodeState {
@@ -36,6 +41,8 @@ struct DecodeState {
 };
 
 __device__ __forceinline__ int decode_class(int bits) { return bits == 2 ? 0 : bits == 3 ? 1 : bits == 4 ? 2 : 3; }
+
+__device__ __forceinline__ int class_bits(int k) { return k == 0 ? 2 : k == 1 ? 3 : k == 2 ? 4 : 8; }
 
 // shared-expert unit u of a list with r row blocks per item (items of 16 slots at T K + 16 j)
 __device__ __forceinline__ Item unit_shared(int u, int r, int E, int T, int K) {
@@ -48,13 +55,36 @@ __device__ __forceinline__ int class_field(uint64_t v, int k) { return int((v >>
 struct DecodePlan {            // LDS
     uint32_t m[PLAN_MAXE];     // token masks
     int start[PLAN_MAXE];      // first slot of each expert
-    uint64_t ig[PLAN_MAXE];    // inclusive scans of the gate_up / down unit counts: 4 classes x 16 bits
-    uint64_t id[PLAN_MAXE];
+    uint64_t it[PLAN_MAXE];    // inclusive scans of the item counts: 4 classes x 16 bits
     int8_t bits[PLAN_MAXE];
-    uint64_t totg, totd;       // class totals
+    uint64_t tot;              // class totals
     int wt_i[4];
-    uint64_t wt_g[4], wt_d[4];
+    uint64_t wt[4];
 };
+
+// log2 of the row blocks per item (16 or 32 over a power of two of strips per wave)
+__device__ __forceinline__ int row_block_shift(bool down, int bits, int fine) {
+    const int s = (down ? 2 : 0) + (bits == 2 ? 2 : bits == 8 ? 0 : 1) - fine;   // log2 of the strips per wave
+    return (down ? 5 : 4) - max(s, 0);
+}
+static_assert(gemm_row_blocks(true, 2) == 2 && gemm_row_blocks(true, 8, 2) == 32 && gemm_row_blocks(false, 8, 1) == 16 &&
+                  gemm_row_blocks(false, 3, 2) == 16,
+              "row_block_shift");
+// units of class k (bits class_bits(k)) per list, and of the whole list, split by fine
+__device__ __forceinline__ int plan_class_units(uint64_t tot, bool down, int k, int fine) {
+    return class_field(tot, k) << row_block_shift(down, class_bits(k), fine);
+}
+__device__ __forceinline__ int plan_units(uint64_t tot, bool down, int fine, int T, int has_shared, int sbits) {
+    int n = has_shared ? ((T + 15) >> 4) << row_block_shift(down, sbits, fine) : 0;
+    for (int k = 0; k < 4; ++k) n += plan_class_units(tot, down, k, fine);
+    return n;
+}
+// the finest split whose units fit `most`
+__device__ __forceinline__ int plan_fine(uint64_t tot, bool down, int most, int T, int has_shared, int sbits) {
+    for (int f = MAX_FINE; f > 0; --f)
+        if (plan_units(tot, down, f, T, has_shared, sbits) <= most) return f;
+    return 0;
+}
 
 // One thread per expert (blockDim 256, E <= 256): P filled, then a barrier. Returns this thread's token mask.
 __device__ __forceinline__ uint32_t decode_plan_scan(int E, const uint32_t* __restrict__ tmask,
@@ -62,84 +92,67 @@ __device__ __forceinline__ uint32_t decode_plan_scan(int E, const uint32_t* __re
     const int e = threadIdx.x, lane = e & 63, w = e >> 6;
     const uint32_t m = e < E ? tmask[e] : 0u;
     const int bw = e < E ? bits[e] : 2;
-    const int c = __popc(m), nit = (c + 15) >> 4, cls = decode_class(bw);
-    const uint64_t vg = uint64_t(nit * gemm_row_blocks(false, bw)) << (16 * cls);
-    const uint64_t vd = uint64_t(nit * gemm_row_blocks(true, bw)) << (16 * cls);
-    // three inclusive scans over the 256 threads in one pass: wave shuffles, then the wave totals
+    const int c = __popc(m), nit = (c + 15) >> 4;
+    // two inclusive scans over the 256 threads in one pass: wave shuffles, then the wave totals
     int incl = wave_incl_scan(c);
-    uint64_t ig = wave_incl_scan(vg), id = wave_incl_scan(vd);
+    uint64_t it = wave_incl_scan(uint64_t(nit) << (16 * decode_class(bw)));
     if (lane == 63) {
         P.wt_i[w] = incl;
-        P.wt_g[w] = ig;
-        P.wt_d[w] = id;
+        P.wt[w] = it;
     }
     __syncthreads();
     for (int i = 0; i < w; ++i) {
         incl += P.wt_i[i];
-        ig += P.wt_g[i];
-        id += P.wt_d[i];
+        it += P.wt[i];
     }
     P.m[e] = m;
     P.start[e] = incl - c;
-    P.ig[e] = ig;
-    P.id[e] = id;
+    P.it[e] = it;
     P.bits[e] = int8_t(bw);
-    if (e == 255) {
-        P.totg = ig;
-        P.totd = id;
-    }
+    if (e == 255) P.tot = it;
     __syncthreads();
     return m;
 }
 
-// total units of the gate_up (down) list
-__device__ __forceinline__ int decode_plan_units(const DecodePlan& P, bool down, int T, int has_shared, int sbits) {
-    const uint64_t tot = down ? P.totd : P.totg;
-    const int ns = has_shared ? (T + 15) >> 4 : 0;
-    return class_field(tot, 0) + class_field(tot, 1) + class_field(tot, 2) + class_field(tot, 3) +
-           ns * gemm_row_blocks(down, sbits);
-}
-
-// Unit u of the gate_up (down) list, from the plan alone (the same unit the dispatch writes at position u).
-__device__ __forceinline__ Item decode_plan_unit(const DecodePlan& P, bool down, int u, int T, int E, int K,
-                                                 int sbits) {
-    const uint64_t tot = down ? P.totd : P.totg;
-    const uint64_t* scan = down ? P.id : P.ig;
+// Unit u of the gate_up (down) list split by fine, from the plan alone (the same unit the dispatch writes at position u).
+// tot: P.tot.
+__device__ __forceinline__ Item decode_plan_unit(const DecodePlan& P, uint64_t tot, bool down, int fine, int u, int T,
+                                                 int E, int K, int sbits) {
     int base = 0;
     for (int k = 0; k < 4; ++k) {
-        const int cnt = class_field(tot, k);
+        const int sh = row_block_shift(down, class_bits(k), fine), cnt = class_field(tot, k) << sh;
         if (u < base + cnt) {
-            const int v = u - base;
-            int lo = 0, hi = E - 1;   // the first expert whose inclusive class-k count exceeds v
+            const int v = (u - base) >> sh;   // item v of the class
+            int lo = 0, hi = E - 1;          // the first expert whose inclusive class-k item count exceeds v
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
-                if (class_field(scan[mid], k) > v) hi = mid;
+                if (class_field(P.it[mid], k) > v) hi = mid;
                 else lo = mid + 1;
             }
-            const int e = lo, bw = P.bits[e], c = __popc(P.m[e]);
-            const int rb = gemm_row_blocks(down, bw), nit = (c + 15) >> 4;
-            const int off = v - (class_field(scan[e], k) - nit * rb), j = off / rb;
-            return Item{e, P.start[e] + 16 * j, min(16, c - 16 * j), off % rb};
+            const int e = lo, c = __popc(P.m[e]), nit = (c + 15) >> 4;
+            const int j = v - (class_field(P.it[e], k) - nit);
+            return Item{e, P.start[e] + 16 * j, min(16, c - 16 * j), (u - base) & ((1 << sh) - 1)};
         }
         base += cnt;
     }
-    return unit_shared(u - base, gemm_row_blocks(down, sbits), E, T, K);
+    return unit_shared(u - base, gemm_row_blocks(down, sbits, fine), E, T, K);
 }
 
 // The written part of the plan. decode_plan_write_expert: expert e's count, start and units of both lists, by the
 // threads i0, i0 + stride, ... decode_plan_write_rest: the shared expert's units and slots, the unit counts, and the
 // placement of every (token, k) pair, by the threads tid, tid + stride, ... P from decode_plan_scan.
-__device__ __forceinline__ void decode_plan_write_expert(const DecodePlan& P, int e, int i0, int stride,
+// fg, fd: the lists' split.
+__device__ __forceinline__ void decode_plan_write_expert(const DecodePlan& P, int e, int i0, int stride, int fg, int fd,
                                                          const DispatchOut& d) {
     const int bw = P.bits[e], c = __popc(P.m[e]), cls = decode_class(bw), nit = (c + 15) >> 4;
-    const int rg = gemm_row_blocks(false, bw), rd = gemm_row_blocks(true, bw);
-    // list positions: the totals of the classes before this one, plus the expert's exclusive count in its class
+    const int rg = gemm_row_blocks(false, bw, fg), rd = gemm_row_blocks(true, bw, fd);
+    // list positions: the units of the classes before this one, plus those of the expert's exclusive items in its class
     int bg = 0, bd = 0;
     for (int k = 0; k < cls; ++k) {
-        bg += class_field(P.totg, k);
-        bd += class_field(P.totd, k);
+        bg += plan_class_units(P.tot, false, k, fg);
+        bd += plan_class_units(P.tot, true, k, fd);
     }
-    const int og = bg + class_field(P.ig[e], cls) - nit * rg, od = bd + class_field(P.id[e], cls) - nit * rd;
+    const int before = class_field(P.it[e], cls) - nit, og = bg + before * rg, od = bd + before * rd;
     if (i0 == 0) {
         d.count[e] = c;
         d.start[e] = P.start[e];
@@ -156,22 +169,21 @@ __device__ __forceinline__ void decode_plan_write_expert(const DecodePlan& P, in
 
 __device__ __forceinline__ void decode_plan_write_rest(const DecodePlan& P, int tid, int stride, int T, int E, int K,
                                                        const int* __restrict__ topk, const float* __restrict__ topw,
-                                                       const DispatchOut& d) {
+                                                       int fg, int fd, const DispatchOut& d) {
     const int sbits = d.has_shared ? d.bits[E] : 8;
     const int ns = d.has_shared ? (T + 15) >> 4 : 0;
-    int bg = 0, bd = 0;
-    for (int k = 0; k < 4; ++k) {
-        bg += class_field(P.totg, k);
-        bd += class_field(P.totd, k);
-    }
-    const int srg = gemm_row_blocks(false, sbits), srd = gemm_row_blocks(true, sbits);
+    const int srg = gemm_row_blocks(false, sbits, fg), srd = gemm_row_blocks(true, sbits, fd);
+    const int ng = plan_units(P.tot, false, fg, T, d.has_shared, sbits), bg = ng - ns * srg;
+    const int nd = plan_units(P.tot, true, fd, T, d.has_shared, sbits), bd = nd - ns * srd;
     for (int u = tid; u < ns * srg; u += stride) d.units_gu[bg + u] = unit_shared(u, srg, E, T, K);
     for (int u = tid; u < ns * srd; u += stride) d.units_dn[bd + u] = unit_shared(u, srd, E, T, K);
     if (tid == 0) {
-        d.n_units[0] = bg + ns * srg;
-        d.n_units[1] = bd + ns * srd;
+        d.n_units[0] = ng;
+        d.n_units[1] = nd;
         d.n_units[2] = 0;
         d.n_units[3] = 0;
+        d.n_units[4] = fg;
+        d.n_units[5] = fd;
     }
     // place every (token, k) pair: slot = the expert's start + the tokens before t that picked it
     for (int p = tid; p < T * K; p += stride) {

@@ -16,6 +16,7 @@
 //                     (engine/moe_i8.cu:219-221)
 //   down    (MODE 1): rows H = 2048, K = I = 512; out Y[slot, h] = w_slot acc (engine/moe_i8.cu:222-231)
 //   products (MODE 2, 3): raw P_g per (token, row, group) in either geometry, for the bit-exactness test.
+#include <algorithm>
 #include <type_traits>
 
 #include "decode_plan.h"
@@ -109,8 +110,8 @@ struct Geo {
     static constexpr int NSB = DOWN_SHAPE ? 1 : 4;       // K = 512 or 2048
     // strips per wave (streamed as one ring) by code width, so that every wave streams about the same bytes
     // (~35 KB): the workgroups of wide codes would otherwise be the tail of the launch
-    template <int BITS>
-    static constexpr int spw() { return gemm_spw(DOWN_SHAPE, BITS); }
+    template <int BITS, int FINE = 0>
+    static constexpr int spw() { return gemm_spw(DOWN_SHAPE, BITS, FINE); }
     static constexpr int SPW_MAX = spw<2>();
 };
 
@@ -149,12 +150,13 @@ struct RowSrc {
     int T, K, E;
 };
 
-template <int BITS, int MODE, int NT, bool PLAN = false>
+// FINE: the units' split (gemm_spw)
+template <int BITS, int MODE, int NT, bool PLAN = false, int FINE = 0>
 __device__ __forceinline__ void gemm_body(const GemmArgs& a, const Item& it, const uint8_t* mat_e, uint8_t* lds,
                                           int row_block, const RowSrc& rs = RowSrc{}) {
-    constexpr int NSB = Geo<MODE>::NSB, SPW = Geo<MODE>::template spw<BITS>(), NSTEP = NSB * SPW;
+    constexpr int NSB = Geo<MODE>::NSB, SPW = Geo<MODE>::template spw<BITS, FINE>(), NSTEP = NSB * SPW;
     constexpr int D = Ring<BITS>::D < NSTEP ? Ring<BITS>::D : NSTEP;
-    static_assert(NSTEP % 4 == 0 && 4 % D == 0, "ring geometry");
+    static_assert(NSTEP % D == 0, "ring geometry");
     constexpr int K = NSB * SB_K, G = K / GROUP, NTOK = 16 * NT, LDQ = K + 16;
     constexpr size_t SBB = sb_bytes(BITS);
     constexpr int ZOFF = BITS == 8 ? 128 : 0;
@@ -468,6 +470,29 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const Item& it, con
     }
 }
 
+// one unit of an expert of `bits`-bit codes, its list split by fine
+template <int MODE, int NT, bool PLAN>
+__device__ __forceinline__ void run_unit(const GemmArgs& a, const Item& it, const uint8_t* mat_e, uint8_t* lds, int bits,
+                                         int fine, const RowSrc& rs = RowSrc{}) {
+    auto go = [&](auto bc, auto fc) {
+        constexpr int B = decltype(bc)::value, F = decltype(fc)::value;
+        // (splits that leave the strips per wave as they are share a body)
+        constexpr int FE = F > 0 && Geo<MODE>::template spw<B, F>() == Geo<MODE>::template spw<B, F - 1>() ? F - 1 : F;
+        constexpr int FF = FE > 0 && Geo<MODE>::template spw<B, FE>() == Geo<MODE>::template spw<B, FE - 1>() ? FE - 1 : FE;
+        gemm_body<B, MODE, NT, PLAN, FF>(a, it, mat_e, lds, it.rb, rs);
+    };
+    auto split = [&](auto bc) {
+        constexpr int F1 = NT > 1 ? 0 : 1, F2 = 2 * F1;   // (the products' lists are never split)
+        if (fine == 0) go(bc, std::integral_constant<int, 0>{});
+        else if (fine == 1) go(bc, std::integral_constant<int, F1>{});
+        else go(bc, std::integral_constant<int, F2>{});
+    };
+    if (bits == 2) split(std::integral_constant<int, 2>{});
+    else if (bits == 3) split(std::integral_constant<int, 3>{});
+    else if (bits == 4) split(std::integral_constant<int, 4>{});
+    else split(std::integral_constant<int, 8>{});
+}
+
 // Persistent: the grid is the number of workgroups that fit the GPU at once; each workgroup takes the work units
 // blockIdx.x, blockIdx.x + gridDim.x, ... (units are ordered longest first, so the long ones start first).
 // Measured at 32 tokens and not kept: units claimed from a device counter as workgroups become free (0.0625 ->
@@ -484,7 +509,7 @@ __global__ void __launch_bounds__(WAVES * 64, NT == 1 ? 3 : 1) expert_gemm(GemmA
     // the unit and the expert's code width and matrix offset are read through the scalar cache (constant address
     // space: the lists are written by earlier kernels only), the width and offset together, so the weight stream
     // starts after two short dependent loads
-    const int n = *a.n_items;
+    const int n = *const_ptr(a.n_items), fine = a.fine ? *const_ptr(a.fine) : 0;
     for (int u = blockIdx.x; u < n; u += gridDim.x) {
         const auto* ip = const_ptr(reinterpret_cast<const int*>(a.items + u));
         const Item it{ip[0], ip[1], ip[2], ip[3]};
@@ -493,10 +518,7 @@ __global__ void __launch_bounds__(WAVES * 64, NT == 1 ? 3 : 1) expert_gemm(GemmA
         asm volatile("" ::"s"(off), "s"(bw4));   // both loads in flight together, before the branch on the width
         const int bits = int(bw4 >> (8 * (it.expert & 3))) << 24 >> 24;
         const uint8_t* mat_e = a.base + off;
-        if (bits == 2) gemm_body<2, MODE, NT>(a, it, mat_e, lds, it.rb);
-        else if (bits == 3) gemm_body<3, MODE, NT>(a, it, mat_e, lds, it.rb);
-        else if (bits == 4) gemm_body<4, MODE, NT>(a, it, mat_e, lds, it.rb);
-        else gemm_body<8, MODE, NT>(a, it, mat_e, lds, it.rb);
+        run_unit<MODE, NT, false>(a, it, mat_e, lds, bits, fine);
         __syncthreads();   // the next unit re-stages the LDS
     }
 }
@@ -510,46 +532,48 @@ __global__ void __launch_bounds__(WAVES * 64, 3) expert_gemm_plan(GemmArgs a, De
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ DecodePlan P;
     decode_plan_scan(p.E, p.tmask, p.d.bits, P);
-    const int sbits = p.d.has_shared ? p.d.bits[p.E] : 8;
+    const int sbits = p.d.has_shared ? __builtin_amdgcn_readfirstlane(int(p.d.bits[p.E])) : 8;
+    // (the class totals in scalar registers: what follows from them is scalar work)
+    const uint64_t tot = (uint64_t(__builtin_amdgcn_readfirstlane(uint32_t(P.tot >> 32))) << 32) |
+                         uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(P.tot)));
+    const int fg = plan_fine(tot, false, p.d.max_gu, p.T, p.d.has_shared, sbits);
+    const int fd = plan_fine(tot, true, p.d.max_dn, p.T, p.d.has_shared, sbits);
     // the writer roles go to the last workgroups, whose units are in the first round only (config 1: 56.8 -> 56.2 us
     // against the first workgroups)
     for (int r = int(gridDim.x - 1 - blockIdx.x); r <= p.E; r += gridDim.x) {
         if (r < p.E) {
-            decode_plan_write_expert(P, r, threadIdx.x, blockDim.x, p.d);
+            decode_plan_write_expert(P, r, threadIdx.x, blockDim.x, fg, fd, p.d);
         } else {
-            decode_plan_write_rest(P, threadIdx.x, blockDim.x, p.T, p.E, p.K, p.topk, p.topw, p.d);
+            decode_plan_write_rest(P, threadIdx.x, blockDim.x, p.T, p.E, p.K, p.topk, p.topw, fg, fd, p.d);
             if (threadIdx.x < p.E) p.tcopy[threadIdx.x] = P.m[threadIdx.x];
         }
     }
-    const int n = decode_plan_units(P, false, p.T, p.d.has_shared, sbits);
+    const int n = plan_units(tot, false, fg, p.T, p.d.has_shared, sbits);
     const RowSrc rs{&P, p.T, p.K, p.E};
     for (int u = blockIdx.x; u < n; u += gridDim.x) {
-        const Item q = decode_plan_unit(P, false, u, p.T, p.E, p.K, sbits);
+        const Item q = decode_plan_unit(P, tot, false, fg, u, p.T, p.E, p.K, sbits);
         const Item it{__builtin_amdgcn_readfirstlane(q.expert), __builtin_amdgcn_readfirstlane(q.slot0),
                       __builtin_amdgcn_readfirstlane(q.ntok), __builtin_amdgcn_readfirstlane(q.rb)};
         const uint64_t off = *const_ptr(a.off + it.expert);
         const int bits = it.expert < p.E ? __builtin_amdgcn_readfirstlane(int(P.bits[it.expert])) : sbits;
         const uint8_t* mat_e = a.base + off;
-        if (bits == 2) gemm_body<2, GEMM_GATE_UP, 1, true>(a, it, mat_e, lds, it.rb, rs);
-        else if (bits == 3) gemm_body<3, GEMM_GATE_UP, 1, true>(a, it, mat_e, lds, it.rb, rs);
-        else if (bits == 4) gemm_body<4, GEMM_GATE_UP, 1, true>(a, it, mat_e, lds, it.rb, rs);
-        else gemm_body<8, GEMM_GATE_UP, 1, true>(a, it, mat_e, lds, it.rb, rs);
+        run_unit<GEMM_GATE_UP, 1, true>(a, it, mat_e, lds, bits, fg, rs);
         __syncthreads();   // the next unit re-stages the LDS
     }
-    // When the gate_up units fit one round, every workgroup then requests the first pf_bytes of down units
+    // When the gate_up units fit one round, every workgroup then requests the first pf_bytes (as much less as they are split) of down units
     // blockIdx.x, blockIdx.x + G, ... (one dword per 64-byte line), so that the down GEMM finds them in the
     // last-level cache (config 0: 0.0429 -> 0.0419 ms per step with 48 KiB; 96 KiB and more slow gate_up down).
     // With a second gate_up round the same requests take bandwidth from it: config 1 (908 units on 768
     // workgroups) went from 0.0540 to 0.0551 ms with 16 KiB requested by the single-unit workgroups.
     const int G = int(gridDim.x);
     if (p.pf_bytes > 0 && n <= G) {
-        const int ndn = decode_plan_units(P, true, p.T, p.d.has_shared, sbits);
+        const int ndn = plan_units(tot, true, fd, p.T, p.d.has_shared, sbits);
         uint32_t sink = 0u;
         for (int d = int(blockIdx.x); d < ndn; d += G) {
-            const Item q = decode_plan_unit(P, true, d, p.T, p.E, p.K, sbits);
+            const Item q = decode_plan_unit(P, tot, true, fd, d, p.T, p.E, p.K, sbits);
             const int e = __builtin_amdgcn_readfirstlane(q.expert), rb = __builtin_amdgcn_readfirstlane(q.rb);
             const int bits = e < p.E ? __builtin_amdgcn_readfirstlane(int(P.bits[e])) : sbits;
-            const int ub = GEMM_WAVES * gemm_spw(true, bits) * int(sb_bytes(bits)), len = min(ub, p.pf_bytes);
+            const int ub = GEMM_WAVES * gemm_spw(true, bits, fd) * int(sb_bytes(bits)), len = min(ub, p.pf_bytes >> fd);
             const uint8_t* src = a.base + *const_ptr(p.d_off + e) + size_t(rb) * ub;
 #pragma unroll 8
             for (int i = int(threadIdx.x) * 64; i < len; i += int(blockDim.x) * 64)
@@ -652,19 +676,30 @@ hipError_t set_attr() {
     return hipFuncSetAttribute(kernel_ptr<MODE, NT>(), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<MODE, NT>());
 }
 
+// workgroups of kernel k resident at once on the whole GPU (0: the query failed)
+int resident_grid(const void* k, int lds) {
+    int dev = 0, cus = 0, per_cu = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, WAVES * 64, lds);
+    return e == hipSuccess ? cus * (per_cu > 0 ? per_cu : 1) : 0;
+}
+template <int MODE, int NT>
+int grid_t() {
+    static int grid = 0;
+    if (!grid) grid = resident_grid(kernel_ptr<MODE, NT>(), lds_bytes<MODE, NT>());
+    return grid;
+}
+int plan_grid() {
+    static int grid = 0;
+    if (!grid) grid = resident_grid(reinterpret_cast<const void*>(&expert_gemm_plan), lds_bytes<GEMM_GATE_UP, 1>());
+    return grid;
+}
+
 template <int MODE, int NT>
 hipError_t launch_t(const GemmArgs& a, int, hipStream_t st) {
-    static int grid = 0;
-    if (!grid) {   // workgroups resident at once on the whole GPU
-        int dev = 0, cus = 0, per_cu = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e == hipSuccess)
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel_ptr<MODE, NT>(), WAVES * 64,
-                                                             lds_bytes<MODE, NT>());
-        if (e != hipSuccess) return e;
-        grid = cus * (per_cu > 0 ? per_cu : 1);
-    }
+    const int grid = grid_t<MODE, NT>();
+    if (!grid) return hipErrorInvalidDevice;
     expert_gemm<MODE, NT><<<grid, WAVES * 64, lds_bytes<MODE, NT>(), st>>>(a);
     return hipGetLastError();
 }
@@ -683,19 +718,12 @@ hipError_t gemm_setup() {
     return hipSuccess;
 }
 
+int expert_grid(int mode) { return mode == GEMM_DOWN ? grid_t<GEMM_DOWN, 1>() : std::min(plan_grid(), grid_t<GEMM_GATE_UP, 1>()); }
+
 hipError_t launch_expert_gemm_plan(const GemmArgs& a, const DecodePlanArgs& p, hipStream_t st) {
     if (p.T < 1 || p.T > 32 || p.E < 1 || p.E > PLAN_MAXE) return hipErrorInvalidValue;
-    static int grid = 0;
-    if (!grid) {   // workgroups resident at once on the whole GPU
-        int dev = 0, cus = 0, per_cu = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e == hipSuccess)
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&expert_gemm_plan),
-                                                             WAVES * 64, lds_bytes<GEMM_GATE_UP, 1>());
-        if (e != hipSuccess) return e;
-        grid = cus * (per_cu > 0 ? per_cu : 1);
-    }
+    const int grid = plan_grid();
+    if (!grid) return hipErrorInvalidDevice;
     expert_gemm_plan<<<grid, WAVES * 64, lds_bytes<GEMM_GATE_UP, 1>(), st>>>(a, p);
     return hipGetLastError();
 }

@@ -25,13 +25,18 @@ struct Item {
 // wave streams about the same bytes (2-bit codes: 4 strips of gate_up, 3/4-bit: 2, 8-bit: 1; down has K/4 and
 // four times the strips).
 constexpr int GEMM_WAVES = 4;
-__host__ __device__ constexpr int gemm_spw(bool down, int bits) {
-    return (down ? 4 : 1) * (bits == 2 ? 4 : bits == 8 ? 1 : 2);
+// A decode step with few units splits them finer: fine = 1, 2 halves, quarters the strips per wave (at least 1). A unit
+// streams its strips one after another, so with the chip mostly idle its length is the launch's: one token of a mixed
+// layer, gate_up 14.6 -> 9.3 us and down 11.4 -> 5.7 us; 8 tokens 17.0 -> 13.7 and 12.1 -> 10.0 us.
+__host__ __device__ constexpr int gemm_spw(bool down, int bits, int fine = 0) {
+    const int s = ((down ? 4 : 1) * (bits == 2 ? 4 : bits == 8 ? 1 : 2)) >> fine;
+    return s > 0 ? s : 1;
 }
 // row blocks (work units per work item) of a gate_up [2I = 1024] or down [H = 2048] matrix
-__host__ __device__ constexpr int gemm_row_blocks(bool down, int bits) {
-    return (down ? 2048 : 1024) / (16 * GEMM_WAVES * gemm_spw(down, bits));
+__host__ __device__ constexpr int gemm_row_blocks(bool down, int bits, int fine = 0) {
+    return (down ? 2048 : 1024) / (16 * GEMM_WAVES * gemm_spw(down, bits, fine));
 }
+constexpr int MAX_FINE = 2;
 constexpr int MAX_UNITS_PER_ITEM = 16;   // gemm_row_blocks(false, 8)
 
 // Tiled GEMM (experts with many tokens): a work unit is a chunk of <= TILED_NTOK slots of one expert and a
@@ -338,6 +343,7 @@ struct GemmArgs {
     const int8_t* bits;         // [E+1]
     const Item* items;          // work units
     const int* n_items;         // device count of work units (the persistent grid loops over them)
+    const int* fine;            // streamed: the units' split (gemm_spw); nullptr: 0
     const int* slot_token;      // gate_up: B row of slot s is token slot_token[s]; nullptr: row = slot
     const int8_t* xq;           // B rows, int8 [rows, K]
     const float* xs;            // [rows, K/128]
@@ -403,6 +409,8 @@ int ensure_gemm_setup();
 int tile_wbytes(int bits);
 size_t packlib_matrix_bytes(int R, int K, int bits);
 
+// resident workgroups of the streamed decode GEMM for mode GEMM_GATE_UP / GEMM_DOWN
+int expert_grid(int mode);
 hipError_t gemm_setup();   // function attributes (dynamic LDS), once per process
 hipError_t launch_expert_gemm(int mode, int nt, const GemmArgs& a, int max_items, hipStream_t st);
 // dense projection at T = a.dense_T <= 32 (K = 2048), split over K (one superblock per wave)
@@ -441,7 +449,8 @@ hipError_t launch_decode_route(const float* part, int nchunks, const float* bias
                                float rscale, float* sig, int32_t* topk, float* topw, uint32_t* blockmax,
                                uint32_t* tmask, int has_shared, const int8_t* bits, int32_t* count, int32_t* start,
                                Item* units_gu, Item* units_dn, int* n_units, int32_t* slot_token, float* slot_weight,
-                               int32_t* tok_slots, const QuantX& qx, int dispatch, hipStream_t st);
+                               int32_t* tok_slots, int max_gu, int max_dn, const QuantX& qx, int dispatch,
+                               hipStream_t st);
 // zero the decode routing state (blockmax, tmask [E]) when no kernel of the step consumed it
 hipError_t launch_zero_decode_state(uint32_t* blockmax, uint32_t* tmask, int E, hipStream_t st);
 hipError_t launch_masks(const int32_t* topk, int T, int E, int K, int block, uint32_t* mask, hipStream_t st);

@@ -360,13 +360,16 @@ __global__ void __launch_bounds__(256) dispatch_kernel(int T, int E, int K, cons
                                                        const float* __restrict__ topw, DecodeState ds, DispatchOut d) {
     __shared__ DecodePlan P;
     decode_plan_scan(E, ds.tmask, d.bits, P);
+    const int sbits = d.has_shared ? d.bits[E] : 8;
+    const int fg = plan_fine(P.tot, false, d.max_gu, T, d.has_shared, sbits);
+    const int fd = plan_fine(P.tot, true, d.max_dn, T, d.has_shared, sbits);
     const int e = threadIdx.x;
     if (e < E) {
         ds.tmask[e] = 0u;
         ds.blockmax[e] = 0u;
-        decode_plan_write_expert(P, e, 0, 1, d);
+        decode_plan_write_expert(P, e, 0, 1, fg, fd, d);
     }
-    decode_plan_write_rest(P, e, 256, T, E, K, topk, topw, d);
+    decode_plan_write_rest(P, e, 256, T, E, K, topk, topw, fg, fd, d);
 }
 
 
@@ -621,6 +624,7 @@ __global__ void __launch_bounds__(PLAN_NT) plan_kernel(const uint32_t* __restric
         n_units[1] = bd;
         n_units[2] = bt;
         n_units[3] = bt;
+        n_units[4] = n_units[5] = 0;   // (the streamed units' split)
     }
     if (!tiled) return;
     // the tiled chunks: tiled_per(c) slots of an expert's c each, the last one shorter (Item.rb unused)
@@ -782,7 +786,8 @@ hipError_t launch_decode_route(const float* part, int nchunks, const float* bias
                                float rscale, float* sig, int32_t* topk, float* topw, uint32_t* blockmax,
                                uint32_t* tmask, int has_shared, const int8_t* bits, int32_t* count, int32_t* start,
                                Item* units_gu, Item* units_dn, int* n_units, int32_t* slot_token, float* slot_weight,
-                               int32_t* tok_slots, const QuantX& qx, int dispatch, hipStream_t st) {
+                               int32_t* tok_slots, int max_gu, int max_dn, const QuantX& qx, int dispatch,
+                               hipStream_t st) {
     if (T > 32 || E > MAXE) return hipErrorInvalidValue;
     const DecodeState ds{blockmax, tmask};
     if (C < E) {
@@ -798,7 +803,7 @@ hipError_t launch_decode_route(const float* part, int nchunks, const float* bias
                                                               topk, topw, ds, qx);
     }
     const DispatchOut d{has_shared, 16, bits, count, start, units_gu, units_dn, n_units, slot_token, slot_weight,
-                        tok_slots};
+                        tok_slots, max_gu, max_dn};
     if (dispatch) dispatch_kernel<<<1, 256, 0, st>>>(T, E, K, topk, topw, ds, d);
     return hipGetLastError();
 }
