@@ -374,7 +374,7 @@ int llmoe_layer_create(const llmoe_layer_desc* desc, const void* blob, size_t bl
     L->items_cap = E + (Tm * K + 15) / 16 + (Tm + 15) / 16 + 2;
     ALLOC(L->units_gu, L->items_cap * MAX_UNITS_PER_ITEM);
     ALLOC(L->units_dn, L->items_cap * MAX_UNITS_PER_ITEM);
-    ALLOC(L->n_units, 6);   // gate_up / down units, tiled chunks (twice), the split of the two streamed lists
+    ALLOC(L->n_units, 6);   // gate_up / down units, tiled chunks (twice), the units of both lists with their split
     L->chunks_cap = E + (Tm * K + TILED_NTOK - 1) / TILED_NTOK + (Tm + TILED_NTOK - 1) / TILED_NTOK + 2;
     if ((5 * L->chunks_cap + 2) * sizeof(uint32_t) > 65536)
         return bail(fail(LLMOE_EINVAL, "max_tokens = %d: more tiled chunks than the planner holds", int(Tm)));
@@ -512,8 +512,7 @@ int experts_impl(llmoe_layer* L, const int8_t* xq, const float* xs, const int32_
     g.slot_weight = L->slot_weight;
     // gate_up: B rows are token rows of x'
     g.items = L->units_gu;
-    g.n_items = L->n_units;
-    g.fine = L->n_units + 4;
+    g.n_items = L->n_units + 4;
     g.off = L->gu_off_d;
     g.slot_token = L->slot_token;
     g.xq = xq; g.xs = xs; g.xsum = xsum;
@@ -551,8 +550,7 @@ int experts_impl(llmoe_layer* L, const int8_t* xq, const float* xs, const int32_
     L->mark(LLMOE_STAGE_FWHT, true, st);
     // down: B rows are slot rows of Z'
     g.items = L->units_dn;
-    g.n_items = L->n_units + 1;
-    g.fine = L->n_units + 5;
+    g.n_items = L->n_units + 5;
     g.off = L->d_off_d;
     g.slot_token = nullptr;
     g.xq = w.zq; g.xs = w.zs; g.xsum = w.zsum;

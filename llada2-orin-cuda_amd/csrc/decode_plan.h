@@ -182,8 +182,8 @@ __device__ __forceinline__ void decode_plan_write_rest(const DecodePlan& P, int 
         d.n_units[1] = nd;
         d.n_units[2] = 0;
         d.n_units[3] = 0;
-        d.n_units[4] = fg;
-        d.n_units[5] = fd;
+        d.n_units[4] = ng | (fg << UNITS_FINE_SHIFT);
+        d.n_units[5] = nd | (fd << UNITS_FINE_SHIFT);
     }
     // place every (token, k) pair: slot = the expert's start + the tokens before t that picked it
     for (int p = tid; p < T * K; p += stride) {

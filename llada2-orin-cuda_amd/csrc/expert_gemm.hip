@@ -481,16 +481,16 @@ __device__ __forceinline__ void run_unit(const GemmArgs& a, const Item& it, cons
         constexpr int FF = FE > 0 && Geo<MODE>::template spw<B, FE>() == Geo<MODE>::template spw<B, FE - 1>() ? FE - 1 : FE;
         gemm_body<B, MODE, NT, PLAN, FF>(a, it, mat_e, lds, it.rb, rs);
     };
-    auto split = [&](auto bc) {
-        constexpr int F1 = NT > 1 ? 0 : 1, F2 = 2 * F1;   // (the products' lists are never split)
-        if (fine == 0) go(bc, std::integral_constant<int, 0>{});
-        else if (fine == 1) go(bc, std::integral_constant<int, F1>{});
-        else go(bc, std::integral_constant<int, F2>{});
+    constexpr int F1 = NT > 1 ? 0 : 1, F2 = 2 * F1;   // (the products' lists are never split)
+    auto widths = [&](auto fc) {
+        if (bits == 2) go(std::integral_constant<int, 2>{}, fc);
+        else if (bits == 3) go(std::integral_constant<int, 3>{}, fc);
+        else if (bits == 4) go(std::integral_constant<int, 4>{}, fc);
+        else go(std::integral_constant<int, 8>{}, fc);
     };
-    if (bits == 2) split(std::integral_constant<int, 2>{});
-    else if (bits == 3) split(std::integral_constant<int, 3>{});
-    else if (bits == 4) split(std::integral_constant<int, 4>{});
-    else split(std::integral_constant<int, 8>{});
+    if (NT > 1 || fine == 0) widths(std::integral_constant<int, 0>{});
+    else if (fine == 1) widths(std::integral_constant<int, F1>{});
+    else widths(std::integral_constant<int, F2>{});
 }
 
 // Persistent: the grid is the number of workgroups that fit the GPU at once; each workgroup takes the work units
@@ -509,7 +509,8 @@ __global__ void __launch_bounds__(WAVES * 64, NT == 1 ? 3 : 1) expert_gemm(GemmA
     // the unit and the expert's code width and matrix offset are read through the scalar cache (constant address
     // space: the lists are written by earlier kernels only), the width and offset together, so the weight stream
     // starts after two short dependent loads
-    const int n = *const_ptr(a.n_items), fine = a.fine ? *const_ptr(a.fine) : 0;
+    const uint32_t nf = uint32_t(*a.n_items);   // (the split beside the count: a second load here cost 0.2 us)
+    const int n = int(nf & UNITS_MASK), fine = int(nf >> UNITS_FINE_SHIFT);
     for (int u = blockIdx.x; u < n; u += gridDim.x) {
         const auto* ip = const_ptr(reinterpret_cast<const int*>(a.items + u));
         const Item it{ip[0], ip[1], ip[2], ip[3]};

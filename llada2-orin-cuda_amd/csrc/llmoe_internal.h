@@ -37,6 +37,8 @@ __host__ __device__ constexpr int gemm_row_blocks(bool down, int bits, int fine 
     return (down ? 2048 : 1024) / (16 * GEMM_WAVES * gemm_spw(down, bits, fine));
 }
 constexpr int MAX_FINE = 2;
+constexpr int UNITS_FINE_SHIFT = 24;
+constexpr uint32_t UNITS_MASK = (1u << UNITS_FINE_SHIFT) - 1u;
 constexpr int MAX_UNITS_PER_ITEM = 16;   // gemm_row_blocks(false, 8)
 
 // Tiled GEMM (experts with many tokens): a work unit is a chunk of <= TILED_NTOK slots of one expert and a
@@ -342,8 +344,8 @@ struct GemmArgs {
     const uint64_t* off;        // [E+1] byte offset of the matrix of each expert (gate_up or down)
     const int8_t* bits;         // [E+1]
     const Item* items;          // work units
-    const int* n_items;         // device count of work units (the persistent grid loops over them)
-    const int* fine;            // streamed: the units' split (gemm_spw); nullptr: 0
+    const int* n_items;         // device count of work units (the persistent grid loops over them); streamed units: with
+                                // their split (gemm_spw) << UNITS_FINE_SHIFT
     const int* slot_token;      // gate_up: B row of slot s is token slot_token[s]; nullptr: row = slot
     const int8_t* xq;           // B rows, int8 [rows, K]
     const float* xs;            // [rows, K/128]

@@ -624,7 +624,8 @@ __global__ void __launch_bounds__(PLAN_NT) plan_kernel(const uint32_t* __restric
         n_units[1] = bd;
         n_units[2] = bt;
         n_units[3] = bt;
-        n_units[4] = n_units[5] = 0;   // (the streamed units' split)
+        n_units[4] = bg;   // (streamed units: not split)
+        n_units[5] = bd;
     }
     if (!tiled) return;
     // the tiled chunks: tiled_per(c) slots of an expert's c each, the last one shorter (Item.rb unused)
