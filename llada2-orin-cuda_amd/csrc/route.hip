@@ -383,9 +383,9 @@ __device__ __forceinline__ void select_top(const uint32_t (&key)[V], int want, b
 // router partials' sum in chunk order, then the sigmoid; with it score_kernel's sigmoid. Meanwhile the last wave finds the
 // block's pool, the C experts with the largest blockmax keys. Then wave 0, four experts per lane, selects the token's top-K
 // of the pool, ranks them among each other and writes them with the routing weights (engine/ops.cu:298-321) and the token
-// masks. All comparisons are (value desc, index asc). Both selections are bit descents over ballots (select_threshold):
-// against bitonic sorts of 64 keys per wave and a merge (and, for the pool, four sorted lists searched per expert):
-// 4.8 -> 4.0 us without the pool, 5.9 -> 4.4 us with it, at 32 tokens.
+// masks. All comparisons are (value desc, index asc). Both selections are bit descents over ballots (select_threshold).
+// Against bitonic sorts of 64 keys per wave and a merge (for the pool, four sorted lists searched per expert): 12.4 -> 10.6
+// us at 2048 tokens, 4.8 and 5.9 us (pool) unchanged at 32, where the launch and the loads are most of it.
 template <bool POOL, bool QA8>
 __global__ void __launch_bounds__(256) select_token_kernel(const float* __restrict__ part, int nchunks,
                                                            const float* __restrict__ sig,

@@ -137,9 +137,11 @@ def _ptr(t) -> int | None:
 
 
 def _stream(stream) -> int | None:
+    """The HIP stream of a call: the given one (a torch stream or a handle), or torch's current stream of the current
+    device. torch.cuda.current_stream() builds a stream object (2.9 us of a 7.7 us call); the handle alone is 0.2 us."""
     if stream is None:
         import torch
-        return torch.cuda.current_stream().cuda_stream
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else stream
 
 
