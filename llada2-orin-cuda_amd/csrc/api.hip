@@ -489,9 +489,7 @@ int llmoe_dispatch(llmoe_layer* L, const int32_t* topk, const float* topw, int T
         HIPCHECK(launch_zero_decode_state(L->blockmax, L->tmask, d.n_experts, st));
     }
     if (int rc = prepare_items(L, T)) return rc;
-    HIPCHECK(hipMemcpyAsync(L->topk, topk, size_t(T) * d.top_k * sizeof(int32_t), hipMemcpyDeviceToDevice, st));
-    HIPCHECK(hipMemcpyAsync(L->topw, topw, size_t(T) * d.top_k * sizeof(float), hipMemcpyDeviceToDevice, st));
-    HIPCHECK(launch_masks(L->topk, T, d.n_experts, d.top_k, d.block, L->mask, st));
+    HIPCHECK(launch_masks(topk, topw, T, d.n_experts, d.top_k, d.block, L->topk, L->topw, L->mask, st));
     return plan_and_place(L, L->topk, L->topw, T, st);
 }
 

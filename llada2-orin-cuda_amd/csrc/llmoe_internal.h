@@ -455,7 +455,9 @@ hipError_t launch_decode_route(const float* part, int nchunks, const float* bias
                                hipStream_t st);
 // zero the decode routing state (blockmax, tmask [E]) when no kernel of the step consumed it
 hipError_t launch_zero_decode_state(uint32_t* blockmax, uint32_t* tmask, int E, hipStream_t st);
-hipError_t launch_masks(const int32_t* topk, int T, int E, int K, int block, uint32_t* mask, hipStream_t st);
+// token masks of externally given routing, and its copy into topk_out / topw_out
+hipError_t launch_masks(const int32_t* topk, const float* topw, int T, int E, int K, int block, int32_t* topk_out,
+                        float* topw_out, uint32_t* mask, hipStream_t st);
 // work units: streamed units_gu / units_dn (n_units[0] / [1], items of <= ntok slots); when `tiled` is set, the
 // chunks of the experts with more than TILED_MIN slots in tunits_gu / tunits_dn (n_units[2] / [3], Item.rb =
 // the chunk's position pre_i) and the work partition of the two tiled grids (g_gu / g_dn workgroups):
