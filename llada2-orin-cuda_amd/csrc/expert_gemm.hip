@@ -471,7 +471,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const Item& it, con
 }
 
 // one unit of an expert of `bits`-bit codes, its list split by fine
-template <int MODE, int NT, bool PLAN>
+template <int MODE, bool PLAN>
 __device__ __forceinline__ void run_unit(const GemmArgs& a, const Item& it, const uint8_t* mat_e, uint8_t* lds, int bits,
                                          int fine, const RowSrc& rs = RowSrc{}) {
     auto go = [&](auto bc, auto fc) {
@@ -479,18 +479,17 @@ __device__ __forceinline__ void run_unit(const GemmArgs& a, const Item& it, cons
         // (splits that leave the strips per wave as they are share a body)
         constexpr int FE = F > 0 && Geo<MODE>::template spw<B, F>() == Geo<MODE>::template spw<B, F - 1>() ? F - 1 : F;
         constexpr int FF = FE > 0 && Geo<MODE>::template spw<B, FE>() == Geo<MODE>::template spw<B, FE - 1>() ? FE - 1 : FE;
-        gemm_body<B, MODE, NT, PLAN, FF>(a, it, mat_e, lds, it.rb, rs);
+        gemm_body<B, MODE, 1, PLAN, FF>(a, it, mat_e, lds, it.rb, rs);
     };
-    constexpr int F1 = NT > 1 ? 0 : 1, F2 = 2 * F1;   // (the products' lists are never split)
     auto widths = [&](auto fc) {
         if (bits == 2) go(std::integral_constant<int, 2>{}, fc);
         else if (bits == 3) go(std::integral_constant<int, 3>{}, fc);
         else if (bits == 4) go(std::integral_constant<int, 4>{}, fc);
         else go(std::integral_constant<int, 8>{}, fc);
     };
-    if (NT > 1 || fine == 0) widths(std::integral_constant<int, 0>{});
-    else if (fine == 1) widths(std::integral_constant<int, F1>{});
-    else widths(std::integral_constant<int, F2>{});
+    if (fine == 0) widths(std::integral_constant<int, 0>{});
+    else if (fine == 1) widths(std::integral_constant<int, 1>{});
+    else widths(std::integral_constant<int, 2>{});
 }
 
 // Persistent: the grid is the number of workgroups that fit the GPU at once; each workgroup takes the work units
@@ -519,7 +518,17 @@ __global__ void __launch_bounds__(WAVES * 64, NT == 1 ? 3 : 1) expert_gemm(GemmA
         asm volatile("" ::"s"(off), "s"(bw4));   // both loads in flight together, before the branch on the width
         const int bits = int(bw4 >> (8 * (it.expert & 3))) << 24 >> 24;
         const uint8_t* mat_e = a.base + off;
-        run_unit<MODE, NT, false>(a, it, mat_e, lds, bits, fine);
+        if constexpr (NT > 1) {
+            // the products' lists are never split; inlined through run_unit's closures, their bodies (accumulators of
+            // four token tiles) kept 304 bytes per lane in scratch: a call on 64 tokens of a 2-bit gate_up took 292 us,
+            // 168 with the direct calls
+            if (bits == 2) gemm_body<2, MODE, NT>(a, it, mat_e, lds, it.rb);
+            else if (bits == 3) gemm_body<3, MODE, NT>(a, it, mat_e, lds, it.rb);
+            else if (bits == 4) gemm_body<4, MODE, NT>(a, it, mat_e, lds, it.rb);
+            else gemm_body<8, MODE, NT>(a, it, mat_e, lds, it.rb);
+        } else {
+            run_unit<MODE, false>(a, it, mat_e, lds, bits, fine);
+        }
         __syncthreads();   // the next unit re-stages the LDS
     }
 }
@@ -558,7 +567,7 @@ __global__ void __launch_bounds__(WAVES * 64, 3) expert_gemm_plan(GemmArgs a, De
         const uint64_t off = *const_ptr(a.off + it.expert);
         const int bits = it.expert < p.E ? __builtin_amdgcn_readfirstlane(int(P.bits[it.expert])) : sbits;
         const uint8_t* mat_e = a.base + off;
-        run_unit<GEMM_GATE_UP, 1, true>(a, it, mat_e, lds, bits, fg, rs);
+        run_unit<GEMM_GATE_UP, true>(a, it, mat_e, lds, bits, fg, rs);
         __syncthreads();   // the next unit re-stages the LDS
     }
     // When the gate_up units fit one round, every workgroup then requests the first pf_bytes (as much less as they are split) of down units
