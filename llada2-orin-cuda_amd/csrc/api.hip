@@ -388,9 +388,12 @@ int llmoe_layer_create(const llmoe_layer_desc* desc, const void* blob, size_t bl
     // units -> 752, 138 down -> 276) 39.3 / 47.1, 32 tokens with the pool (280 -> 528, 140 -> 280) 42.9 / 50.4. Beyond:
     // two rounds of gate_up units 43.9; 560 down units 43.6; 384 down units (4-bit experts, 192 unsplit) 42.9 / 42.5. The
     // lists hold at least 64 MAX_UNITS_PER_ITEM units.
-    L->max_gu = std::min<long>(expert_grid(GEMM_GATE_UP), long(L->items_cap) * MAX_UNITS_PER_ITEM);
-    L->max_dn = std::min<long>(long(expert_grid(GEMM_DOWN)) * 5 / 12, long(L->items_cap) * MAX_UNITS_PER_ITEM);
-    if (L->max_gu < 1 || L->max_dn < 1) return bail(fail(LLMOE_EHIP, "GEMM occupancy query failed"));
+    int grid_gu = 0, grid_dn = 0;
+    hipError_t ge = expert_grid(GEMM_GATE_UP, &grid_gu);
+    if (ge == hipSuccess) ge = expert_grid(GEMM_DOWN, &grid_dn);
+    if (ge != hipSuccess) return bail(fail(LLMOE_EHIP, "GEMM occupancy query: %s", hipGetErrorString(ge)));
+    L->max_gu = std::min<long>(grid_gu, long(L->items_cap) * MAX_UNITS_PER_ITEM);
+    L->max_dn = std::min<long>(long(grid_dn) * 5 / 12, long(L->items_cap) * MAX_UNITS_PER_ITEM);
     ALLOC(L->tstart, size_t(L->g_gu + L->g_dn + 2));
     ALLOC(L->slot_token, S);
     ALLOC(L->slot_weight, S);

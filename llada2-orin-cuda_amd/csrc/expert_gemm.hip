@@ -686,30 +686,35 @@ hipError_t set_attr() {
     return hipFuncSetAttribute(kernel_ptr<MODE, NT>(), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<MODE, NT>());
 }
 
-// workgroups of kernel k resident at once on the whole GPU (0: the query failed)
-int resident_grid(const void* k, int lds) {
+// grid: the workgroups of kernel k resident at once on the whole GPU (asked once: a known grid stays)
+hipError_t resident_grid(const void* k, int lds, int& grid) {
+    if (grid) return hipSuccess;
     int dev = 0, cus = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, WAVES * 64, lds);
-    return e == hipSuccess ? cus * (per_cu > 0 ? per_cu : 1) : 0;
+    if (e == hipSuccess) grid = cus * (per_cu > 0 ? per_cu : 1);
+    return e;
 }
 template <int MODE, int NT>
-int grid_t() {
+hipError_t grid_t(int& g) {
     static int grid = 0;
-    if (!grid) grid = resident_grid(kernel_ptr<MODE, NT>(), lds_bytes<MODE, NT>());
-    return grid;
+    const hipError_t e = resident_grid(kernel_ptr<MODE, NT>(), lds_bytes<MODE, NT>(), grid);
+    g = grid;
+    return e;
 }
-int plan_grid() {
+hipError_t plan_grid(int& g) {
     static int grid = 0;
-    if (!grid) grid = resident_grid(reinterpret_cast<const void*>(&expert_gemm_plan), lds_bytes<GEMM_GATE_UP, 1>());
-    return grid;
+    const hipError_t e =
+        resident_grid(reinterpret_cast<const void*>(&expert_gemm_plan), lds_bytes<GEMM_GATE_UP, 1>(), grid);
+    g = grid;
+    return e;
 }
 
 template <int MODE, int NT>
 hipError_t launch_t(const GemmArgs& a, int, hipStream_t st) {
-    const int grid = grid_t<MODE, NT>();
-    if (!grid) return hipErrorInvalidDevice;
+    int grid = 0;
+    if (const hipError_t e = grid_t<MODE, NT>(grid); e != hipSuccess) return e;
     expert_gemm<MODE, NT><<<grid, WAVES * 64, lds_bytes<MODE, NT>(), st>>>(a);
     return hipGetLastError();
 }
@@ -728,12 +733,18 @@ hipError_t gemm_setup() {
     return hipSuccess;
 }
 
-int expert_grid(int mode) { return mode == GEMM_DOWN ? grid_t<GEMM_DOWN, 1>() : std::min(plan_grid(), grid_t<GEMM_GATE_UP, 1>()); }
+hipError_t expert_grid(int mode, int* grid) {
+    int g = 0, p = 0;
+    hipError_t e = mode == GEMM_DOWN ? grid_t<GEMM_DOWN, 1>(g) : grid_t<GEMM_GATE_UP, 1>(g);
+    if (e == hipSuccess && mode == GEMM_GATE_UP) e = plan_grid(p);
+    *grid = mode == GEMM_GATE_UP ? std::min(g, p) : g;
+    return e;
+}
 
 hipError_t launch_expert_gemm_plan(const GemmArgs& a, const DecodePlanArgs& p, hipStream_t st) {
     if (p.T < 1 || p.T > 32 || p.E < 1 || p.E > PLAN_MAXE) return hipErrorInvalidValue;
-    const int grid = plan_grid();
-    if (!grid) return hipErrorInvalidDevice;
+    int grid = 0;
+    if (const hipError_t e = plan_grid(grid); e != hipSuccess) return e;
     expert_gemm_plan<<<grid, WAVES * 64, lds_bytes<GEMM_GATE_UP, 1>(), st>>>(a, p);
     return hipGetLastError();
 }

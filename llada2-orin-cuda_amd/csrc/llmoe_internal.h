@@ -411,8 +411,8 @@ int ensure_gemm_setup();
 int tile_wbytes(int bits);
 size_t packlib_matrix_bytes(int R, int K, int bits);
 
-// resident workgroups of the streamed decode GEMM for mode GEMM_GATE_UP / GEMM_DOWN
-int expert_grid(int mode);
+// *grid: resident workgroups of the streamed decode GEMM for mode GEMM_GATE_UP / GEMM_DOWN
+hipError_t expert_grid(int mode, int* grid);
 hipError_t gemm_setup();   // function attributes (dynamic LDS), once per process
 hipError_t launch_expert_gemm(int mode, int nt, const GemmArgs& a, int max_items, hipStream_t st);
 // dense projection at T = a.dense_T <= 32 (K = 2048), split over K (one superblock per wave)

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import struct
 from pathlib import Path
 
 import numpy as np
@@ -147,3 +148,22 @@ def test_null_layer_rejected(lib, name):
     rc = _NULL_LAYER_CALLS[name](getattr(lib, name))
     assert rc == -1, f"{name} returned {rc}"   # LLMOE_EINVAL
     assert b"null layer" in lib.llmoe_last_error(), lib.llmoe_last_error()
+
+
+def test_launch_reports_the_runtimes_error(lib):
+    """Without a device the streamed GEMMs' launches return what the runtime says (hipErrorNoDevice), not an error of
+    their own: the message of a failed call is made from it."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    n = ctypes.c_int()
+    want = hip.hipGetDeviceCount(ctypes.byref(n))
+    if want == 0 and n.value > 0:
+        pytest.skip("has a GPU")
+    assert want != 0
+    args = ctypes.create_string_buffer(4096)   # zeros: never read without a device
+    gemm = getattr(lib, "_ZN5llmoe18launch_expert_gemmEiiRKNS_8GemmArgsEiP12ihipStream_t")
+    for mode, nt in ((0, 1), (1, 1), (2, 4), (3, 4)):
+        assert gemm(mode, nt, args, 0, None) == want, mode
+    plan = ctypes.create_string_buffer(4096)
+    plan[0:8] = struct.pack("<ii", 1, 64)      # T, E
+    f = getattr(lib, "_ZN5llmoe23launch_expert_gemm_planERKNS_8GemmArgsERKNS_14DecodePlanArgsEP12ihipStream_t")
+    assert f(args, plan, None) == want
