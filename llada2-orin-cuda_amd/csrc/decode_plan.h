@@ -63,13 +63,18 @@ struct DecodePlan {            // LDS
 };
 
 // log2 of the row blocks per item (16 or 32 over a power of two of strips per wave)
-__device__ __forceinline__ int row_block_shift(bool down, int bits, int fine) {
+__host__ __device__ constexpr int row_block_shift(bool down, int bits, int fine) {
     const int s = (down ? 2 : 0) + (bits == 2 ? 2 : bits == 8 ? 0 : 1) - fine;   // log2 of the strips per wave
-    return (down ? 5 : 4) - max(s, 0);
+    return (down ? 5 : 4) - (s > 0 ? s : 0);
 }
-static_assert(gemm_row_blocks(true, 2) == 2 && gemm_row_blocks(true, 8, 2) == 32 && gemm_row_blocks(false, 8, 1) == 16 &&
-                  gemm_row_blocks(false, 3, 2) == 16,
-              "row_block_shift");
+constexpr bool row_block_shift_agrees() {
+    for (int down = 0; down < 2; ++down)
+        for (int bits : {2, 3, 4, 8})
+            for (int fine = 0; fine <= MAX_FINE; ++fine)
+                if (1 << row_block_shift(down, bits, fine) != gemm_row_blocks(down, bits, fine)) return false;
+    return true;
+}
+static_assert(row_block_shift_agrees(), "list positions (row_block_shift) against the units written (gemm_row_blocks)");
 // units of class k (bits class_bits(k)) per list, and of the whole list, split by fine
 __device__ __forceinline__ int plan_class_units(uint64_t tot, bool down, int k, int fine) {
     return class_field(tot, k) << row_block_shift(down, class_bits(k), fine);
