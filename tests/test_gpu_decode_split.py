@@ -18,6 +18,11 @@ pytestmark = pytest.mark.gpu
     (20, 2, True, 16, (2, 2)),           # a pool of 16: items of 16 slots, two per busy expert
     (17, 3, True, 40, (2, 0)),           # two shared items; 3-bit gate_up units halved (their most), down unsplit
     (32, "mixed", True, 256, (0, 0)),    # about 160 experts: no split
+    (8, 2, False, 256, (1, 1)),          # gate_up between the bounds: halved, not quartered
+    (32, "mixed", True, 48, (1, 1)),
+    (4, 3, False, 256, (2, 1)),
+    (2, 8, False, 256, (2, 1)),
+    (4, 8, True, 256, (2, 0)),           # the finest gate_up beside unsplit down units
 ])
 def test_split_units_match_oracle(gpu, T, mix, shared, pool, split):
     import torch
