@@ -163,7 +163,13 @@ typedef struct {
     int32_t* slot_token; float* slot_weight;           /*                              [S] */
     int32_t* tok_slots;                                /* [T, K + 1] (last: shared slot, -1 if none) */
     int32_t* items; int32_t* n_items;                  /* gate_up work units {expert, slot0, ntok, row block};
-                                                          n_items[0] / [1]: gate_up / down unit counts */
+                                                          n_items[0] / [1]: gate_up / down unit counts; [4] / [5]:
+                                                          the same count | split << 24 of the streamed units. A
+                                                          unit covers 64 s rows (row block * 64 s ...), s the
+                                                          strips per wave: gate_up 4, 2, 2, 1 and down 16, 8, 8, 4
+                                                          of 2, 3, 4, 8-bit codes, halved once (split 1) or twice
+                                                          (split 2) but at least 1; only a decode step of the
+                                                          layer's own routing splits. [2] / [3]: tiled chunks */
     uint16_t* Z;                                       /* fp16 SiLU(g) u               [S, I] */
     int8_t* zq; float* zs; int32_t* zsum;              /* A8(Z H512)                   [S, I], [S, I/128] */
     float* Y;                                          /* weighted expert outputs      [S, H]
