@@ -383,11 +383,11 @@ int llmoe_layer_create(const llmoe_layer_desc* desc, const void* blob, size_t bl
     L->g_gu = tiled_grid(GEMM_GATE_UP);
     L->g_dn = tiled_grid(GEMM_DOWN);
     if (L->g_gu < 1 || L->g_dn < 1) return bail(fail(LLMOE_EHIP, "tiled GEMM occupancy query failed"));
-    // Decode units are split finer while they run in one round (gate_up), or at 5/4 units per CU (down: every unit
-    // transforms its item's Z rows again). us a layer, split against not: one token 31.4 / 43.2, 8 tokens (276 gate_up
-    // units -> 752, 138 down -> 276) 39.3 / 47.1, 32 tokens with the pool (280 -> 528, 140 -> 280) 42.9 / 50.4. Beyond:
-    // two rounds of gate_up units 43.9; 560 down units 43.6; 384 down units (4-bit experts, 192 unsplit) 42.9 / 42.5. The
-    // lists hold at least 64 MAX_UNITS_PER_ITEM units.
+    // Decode units are split finer while they run in one round (gate_up), or in 5/12 of one (down, where every unit
+    // transforms its item's Z rows again; with three resident workgroups per CU that is 5/4 units per CU). us a layer,
+    // split against not: one token 31.4 / 43.2, 8 tokens (276 gate_up units -> 752, 138 down -> 276) 39.3 / 47.1, 32
+    // tokens with the pool (280 -> 528, 140 -> 280) 42.9 / 50.4. Beyond: two rounds of gate_up units 43.9; 560 down units
+    // 43.6; 384 down units (4-bit experts, 192 unsplit) 42.9 / 42.5. The lists hold at least 64 MAX_UNITS_PER_ITEM units.
     int grid_gu = 0, grid_dn = 0;
     hipError_t ge = expert_grid(GEMM_GATE_UP, &grid_gu);
     if (ge == hipSuccess) ge = expert_grid(GEMM_DOWN, &grid_dn);

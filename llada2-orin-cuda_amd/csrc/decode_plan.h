@@ -7,13 +7,13 @@
 // blocks by code width, ordered by class -- 2, 3, 4, 8-bit experts (expert order within a class), then the shared
 // expert's -- so the longest units start first.
 //
-// Every workgroup of 256 threads can build the plan in LDS (one thread per expert: three scans), and any of them
+// Every workgroup of 256 threads can build the plan in LDS (one thread per expert: two scans), and any of them
 // can then name unit u of the gate_up list without the list in memory: the class from the class totals, the
 // expert by binary search on the class's inclusive scan, then the item and row block.
 //
 // Few units leave most of the chip idle while each streams its strips one after another, so the plan splits the units
-// of a list finer (half, a quarter of the strips per wave) as long as they still fit the resident workgroups in one
-// round (DispatchOut::max_gu, max_dn).
+// of a list finer (half, a quarter of the strips per wave) as long as there are no more of them than DispatchOut::max_gu
+// (gate_up: one round of the resident workgroups) and max_dn (down: 5/12 of a round, as each repeats its item's FWHT).
 #pragma once
 #include "llmoe_internal.h"
 

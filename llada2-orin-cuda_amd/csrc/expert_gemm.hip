@@ -296,8 +296,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const Item& it, con
     static_assert(!ZBUF || UROWS / 2 * 16 * 2 <= ZBUF_BYTES, "Z buffer");
     uint32_t* zlds = reinterpret_cast<uint32_t*>(lds + ybuf_offset<MODE, NT>());
 
-    // the wave's NSTEP superblocks (SPW strips of NSB each) are streamed as one ring (slot of step u = u % D). The steps are unrolled at compile time: across a loop back-edge the compiler would wait for every
-    // outstanding load, and the prefetch would not overlap.
+    // the wave's NSTEP superblocks (SPW strips of NSB each) are streamed as one ring (slot of step u = u % D). The steps
+    // are unrolled at compile time: across a loop back-edge the compiler would wait for every outstanding load, and the
+    // prefetch would not overlap.
     static_for<0, NSTEP>([&](auto uc) {
         constexpr int u = decltype(uc)::value;
         Step<BITS>& cur = ring[u % D];
@@ -570,10 +571,10 @@ __global__ void __launch_bounds__(WAVES * 64, 3) expert_gemm_plan(GemmArgs a, De
         run_unit<GEMM_GATE_UP, true>(a, it, mat_e, lds, bits, fg, rs);
         __syncthreads();   // the next unit re-stages the LDS
     }
-    // When the gate_up units fit one round, every workgroup then requests the first pf_bytes (as much less as they are split) of down units
-    // blockIdx.x, blockIdx.x + G, ... (one dword per 64-byte line), so that the down GEMM finds them in the
-    // last-level cache (config 0: 0.0429 -> 0.0419 ms per step with 48 KiB; 96 KiB and more slow gate_up down).
-    // With a second gate_up round the same requests take bandwidth from it: config 1 (908 units on 768
+    // When the gate_up units fit one round, every workgroup then requests the first pf_bytes (pf_bytes >> fd of units
+    // split by fd) of down units blockIdx.x, blockIdx.x + G, ... (one dword per 64-byte line), so that the down GEMM
+    // finds them in the last-level cache (config 0: 0.0429 -> 0.0419 ms per step with 48 KiB; 96 KiB and more slow
+    // gate_up down). With a second gate_up round the same requests take bandwidth from it: config 1 (908 units on 768
     // workgroups) went from 0.0540 to 0.0551 ms with 16 KiB requested by the single-unit workgroups.
     const int G = int(gridDim.x);
     if (p.pf_bytes > 0 && n <= G) {

@@ -27,7 +27,9 @@ struct Item {
 constexpr int GEMM_WAVES = 4;
 // A decode step with few units splits them finer: fine = 1, 2 halves, quarters the strips per wave (at least 1). A unit
 // streams its strips one after another, so with the chip mostly idle its length is the launch's: one token of a mixed
-// layer, gate_up 14.6 -> 9.3 us and down 11.4 -> 5.7 us; 8 tokens 17.0 -> 13.7 and 12.1 -> 10.0 us.
+// layer, gate_up 15.6 -> 9.9 us and down 12.0 -> 5.9 us; 19 tokens with a pool of 48 18.7 -> 15.9 and 13.6 -> 10.5 us
+// (kernel trace, against units that are not split). MAX_FINE = 2 brings gate_up to one strip per wave at every width, and
+// down to 4, 2, 2, 1 (2, 3, 4, 8-bit); more for down is not built.
 __host__ __device__ constexpr int gemm_spw(bool down, int bits, int fine = 0) {
     const int s = ((down ? 4 : 1) * (bits == 2 ? 4 : bits == 8 ? 1 : 2)) >> fine;
     return s > 0 ? s : 1;

@@ -116,9 +116,9 @@ __global__ void __launch_bounds__(256) router_decode_kernel(const float* __restr
 // reads the k of four MFMAs (its k are congruent mod 4) as 16 bytes (row stride 68: conflict-free); Wr operands come
 // straight from global memory (64 contiguous bytes per k). A stage's loads are in flight during the stage before.
 // Experts are the MFMA rows, so a lane ends with four consecutive experts of one token.
-// What bounds it: the f32 MFMA issue (28 us of 4096 tokens' 59 at 2.4 GHz; vector work does not overlap f32 MFMAs, so
-// the A8 and the addressing add to it). Against vector fma chains on 64 x 64 tiles in LDS: 15.1 -> 10.5 us at 512
-// tokens, 93 -> 59 us at 4096.
+// What bounds it: the f32 MFMA issue (28 us of 4096 tokens' 52 at 2.4 GHz; vector work does not overlap f32 MFMAs, so
+// the A8 and the addressing add to it). Against vector fma chains on 64 x 64 tiles in LDS, by kernel traces on one box:
+// 13.8 -> 9.4 us at 512 tokens, 83 -> 52 us at 4096.
 typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int RM_KS = 64, RM_STRIDE = RM_KS + 4;
 template <int M>
@@ -379,13 +379,15 @@ __device__ __forceinline__ void select_top(const uint32_t (&key)[V], int want, b
     }
 }
 
-// Selection, one token per workgroup (engine/ops.cu:256-327). Thread e scores expert e: without the pool the logit is the
-// router partials' sum in chunk order, then the sigmoid; with it score_kernel's sigmoid. Meanwhile the last wave finds the
-// block's pool, the C experts with the largest blockmax keys. Then wave 0, four experts per lane, selects the token's top-K
-// of the pool, ranks them among each other and writes them with the routing weights (engine/ops.cu:298-321) and the token
-// masks. All comparisons are (value desc, index asc). Both selections are bit descents over ballots (select_threshold).
-// Against bitonic sorts of 64 keys per wave and a merge (for the pool, four sorted lists searched per expert): 12.4 -> 10.6
-// us at 2048 tokens, 4.8 and 5.9 us (pool) unchanged at 32, where the launch and the loads are most of it.
+// Selection, one token per workgroup (engine/ops.cu:256-327). Thread e scores expert e: without the pool the logit is
+// the router partials' sum in chunk order, then the sigmoid; with it score_kernel's sigmoid. Meanwhile the last wave
+// finds the block's pool, the C experts with the largest blockmax keys. Then wave 0, four experts per lane, selects the
+// token's top-K of the pool, ranks them among each other and writes them with the routing weights
+// (engine/ops.cu:298-321) and the token masks. All comparisons are (value desc, index asc). Both selections are bit
+// descents over ballots (select_threshold).
+// Against bitonic sorts of 64 keys per wave and a merge (for the pool, four sorted lists searched per expert), by kernel
+// traces on one box: 11.5 -> 9.8 us at 2048 tokens, 15.2 -> 11.4 at 4096 (2 % of such a layer). At 32 tokens 4.7 us and
+// with the pool 5.8 us either way, where the launch and the loads are most of it: there it is the one form for both.
 template <bool POOL, bool QA8>
 __global__ void __launch_bounds__(256) select_token_kernel(const float* __restrict__ part, int nchunks,
                                                            const float* __restrict__ sig,
@@ -476,9 +478,10 @@ __global__ void __launch_bounds__(256) select_token_kernel(const float* __restri
 }
 
 
-// Token masks of externally given routing, and the layer's copy of it (the caller's arrays are free once the call's work
-// is done). Bound by launch latency: with the copies as two copy commands of the runtime, those took 4.0 us each, more
-// than this kernel's 3.2 us. The copies may be the given arrays themselves. grid nb, 256 threads.
+// Token masks of externally given routing, and the layer's copy of it (the caller's arrays are free once the call's
+// work is done). Bound by launch latency: two copy commands of the runtime took 4.0 us each beside this kernel's 3.9 us;
+// with the copies in the kernel it takes 4.6 us (77 tokens). The copies may be the given arrays themselves. grid nb, 256
+// threads.
 __global__ void __launch_bounds__(256) masks_kernel(const int* topk, const float* topw, int T, int E, int K, int block,
                                                     int* topk_out, float* topw_out, uint32_t* __restrict__ mask) {
     __shared__ uint32_t tmask[MAXE];
@@ -786,7 +789,9 @@ hipError_t launch_router_logits(const float* x, const float* Wr, int T, int H, i
                                 float* qs, int* qsum, hipStream_t st) {
     if (T <= 32) {
         router_decode_kernel<<<dim3(E / RD_EW, 1, ROUTER_KC), 256, RD_LDS, st>>>(x, Wr, T, H, E, part, q, qs, qsum);
-    } else if (T <= 256) {   // 32 x 32 tiles: at 256 tokens 512 workgroups (64 x 64: 128, half of the CUs)
+    } else if (T <= 256) {
+        // 32 x 32 tiles: with 256 experts 512 workgroups at 256 tokens (64 x 64: 128, half of the CUs). The line was
+        // measured at 256 experts only; fewer give fewer workgroups at either size.
         router_mfma_kernel<1><<<dim3(E / 32, (T + 31) / 32, ROUTER_KC), 256, rm_lds<1>(), st>>>(x, Wr, T, H, E, part, q,
                                                                                                qs, qsum);
     } else {
