@@ -381,7 +381,7 @@ def dense_config(llmoe, synth, torch, R, bits, T, steps, warmup, nmat=40):
     y = torch.empty((T, R), dtype=torch.float32, device=dev)
     dt = time_steps(lambda i: Ds[i % nmat].forward(xq, xs, xsum, out=y), steps, warmup)
     # GPU time per projection: one projection per matrix captured back to back in a HIP graph, replayed (a Python
-    # call per projection costs more host time than a 32-token projection takes on the GPU)
+    # call per projection takes the host about as long as a 32-token projection takes the GPU)
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):
